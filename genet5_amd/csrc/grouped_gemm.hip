@@ -24,15 +24,15 @@
 // source chunk, so that 16-lane groups of the fragment reads hit 16 distinct
 // bank groups of the 64-bank LDS.  Two LDS stages.  Fragments are read two
 // substeps ahead into three register slots, so a stage buffer is free two
-// substeps before its k-step ends; its refill (the stage two k-steps ahead) is
-// issued one DMA instruction after every other MFMA over those substeps, which
-// keeps the texture path busy without stalling the matrix core (issuing a
-// stage's 16 instructions in one burst stalled the MFMA stream for about as
-// long as the DMA took).  The in-place GEMMs (down and the backward's, whose A
-// rows come from HBM rather than the small gathered x) keep a third A stage in
-// the epilogue region and issue A three k-steps ahead (down 9 % faster); the
-// SwiGLU GEMMs do the same for B, the weight tiles, which stream from beyond
-// the L2 (the training forward's gate|up 5 % faster, the inference one even).
+// substeps before its k-step ends, when its refill (the stage two k-steps ahead)
+// may start.  The operand that streams from beyond the L2 (the in-place GEMMs'
+// A rows, the SwiGLU GEMMs' weight tiles) has a third buffer in the epilogue
+// region, free for the whole k-step: its 8 DMA instructions go out over the
+// k-step's first half, the other operand's 8 over the second, one after every
+// fourth MFMA.  The DMA path takes about 45 B per clock and CU; all 16 in the
+// second half asked 64 of it and the in-order waves' MFMA streams stalled behind
+// them (36,400 tokens, outputs the same bit for bit: the layer 957 -> 940 us, the
+// training step 3,329 -> 3,281 us; 4,550 tokens 189 -> 187 us).
 //
 // Scheduling: expert row counts live on the device (offsets[]); the grid is
 // one workgroup per CU, and each workgroup walks a list of tiles derived from
@@ -282,19 +282,21 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
   // The gate|up GEMMs gather token rows through perm; the others read the
   // expert-contiguous A rows in place.
   constexpr bool GATHER = MODE != 0 && MODE != 4;
-  // Three A stages (MODE 0 with three fragment slots): the epilogue region,
+  // Three A buffers (MODE 0 / 4 with three fragment slots): the epilogue region,
   // which is exactly one A stage (wave w's DMA slice of it is wave w's own
-  // region), doubles as A buffer 2, so A is issued three k-steps ahead and B
-  // two.  A buffers rotate with the k-step mod 3 (tiles start at 0 mod 3, so
-  // every tile's last step reads its A from the epilogue region: the next
-  // tile's third A stage goes out after the epilogue), B buffers mod 2.
+  // region), doubles as A buffer 2, so step g's free A buffer is refilled (stage
+  // g + 2) from the step's start and B's after the step's barrier.  A buffers
+  // rotate with the k-step mod 3 (tiles start at 0 mod 3, so every tile's last
+  // step reads its A from the epilogue region, which the next tile's first step
+  // refills after the epilogue), B buffers mod 2.
   constexpr bool A3 = G5_A3 && (MODE == 0 || MODE == 4) && NSLOT == 3 && S == 2 &&
                       A_BYTES == 4 * EPI;
-  // Three B stages (the SwiGLU modes, whose weight tiles are the operand that
+  // Three B buffers (the SwiGLU modes, whose weight tiles are the operand that
   // streams from beyond the L2): the same scheme with the roles swapped, B
-  // buffer 2 being the epilogue region, B issued three k-steps ahead and A
-  // two.  The next tile's gathered rows then travel through a VGPR instead of
-  // that region.
+  // buffer 2 being the epilogue region.  The next tile's gathered rows then
+  // travel through a VGPR instead of that region; the step whose barrier reads
+  // it (the tile's last but one) waits for every load there, so it issues both
+  // operands after the barrier (LATE).
   constexpr bool B3 = G5_B3 && SWIGLU && NSLOT == 3 && S == 2 &&
                       B_BYTES == 4 * EPI;
   auto decode_unit = [&](int i, TileCoord& tc) {
@@ -488,8 +490,7 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
           *reinterpret_cast<const bf16x8*>(Bs + b_row + (f - MB) * 32 * RB + pc);
   };
 
-  // Prologue: stages 0 .. S-1 of the first tile (nk >= S); A3: A0 B0 A1 B1 A2
-  // (nk >= 6).
+  // Prologue: stages 0 .. S-1 of the first tile (nk >= S).
   if constexpr (A3) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -498,10 +499,8 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
 #pragma unroll
       for (int j = 0; j < BI; ++j) issue_b(bbuf3(st), b_cur, st * BK, j);
     }
-#pragma unroll
-    for (int q = 0; q < AI; ++q) issue_a(abuf3(2), a_cur, 2 * BK, q);
-    wait_vmcnt<PER + AI>();  // A0 and B0 landed
-  } else if constexpr (B3) {  // A0 B0 A1 B1 B2
+    wait_vmcnt<PER>();  // A0 and B0 landed
+  } else if constexpr (B3) {
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
@@ -509,9 +508,7 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
 #pragma unroll
       for (int j = 0; j < BI; ++j) issue_b(bbuf3b(st), b_cur, st * BK, j);
     }
-#pragma unroll
-    for (int j = 0; j < BI; ++j) issue_b(bbuf3b(2), b_cur, 2 * BK, j);
-    wait_vmcnt<PER + BI>();  // A0 and B0 landed
+    wait_vmcnt<PER>();  // A0 and B0 landed
   } else {
 #pragma unroll
     for (int st = 0; st < S; ++st)
@@ -538,13 +535,17 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
   // One k-step (KS substeps of 16 k) of the current tile.  FIRST: the tile's
   // first step (zero accumulator input); LAST: its last step (the next step's
   // first fragments are read after the epilogue instead).  At the start of the
-  // last substep the wave waits for step g + 1's stage, syncs (every wave is
-  // done reading buffer g % S), and then refills that buffer with stage g + S,
-  // one DMA instruction after every other MFMA of the substep.
-  auto kstep = [&](auto first_c, auto last_c, auto phase_c, int kt) __attribute__((always_inline)) {
+  // substep BS the wave waits for step g + 1's stage, syncs (every wave is
+  // done reading buffer g % S), and then refills that buffer with stage g + S;
+  // the three-buffer operand's part of stage g + S goes out before it.
+  auto kstep = [&](auto first_c, auto last_c, auto phase_c, int kt,
+                   auto late_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value;
     constexpr bool LAST = decltype(last_c)::value;
     constexpr int PHASE = decltype(phase_c)::value;  // gstep % 3 when NSLOT == 3
+    constexpr bool LATE = decltype(late_c)::value;
+    // the three-buffer operand's refill goes out before the barrier
+    constexpr bool EARLY = (A3 || B3) && !LATE;
     auto slot = [](int ks) { return NSLOT == 2 ? (ks & 1) : (PHASE * KS + ks) % 3; };
     const int cb = gstep % S;
     const int nb = (gstep + 1) % S;
@@ -572,34 +573,28 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
     const char* const b_nxt_v = b_nxt;
     const char* a_fill = use_nxt ? a_nxt_v : a_cur_v;
     const char* b_fill = use_nxt ? b_nxt_v : b_cur_v;
-    // A3: B refills as above (stage kt + 2); A refills with stage kt + 3,
-    // except on the tile's last step, whose A buffer the epilogue uses.  B3:
-    // the same with A and B swapped.
-    const int ka_fill = kt + 3;
-    const bool afill_cur = ka_fill < nk;
-    const int k0_afill = afill_cur ? ka_fill * BK : (has_nxt ? (ka_fill - nk) * BK : 0);
-    const char* a3_fill = (!afill_cur && has_nxt) ? a_nxt_v : a_cur_v;
-    const char* b3_fill = (!afill_cur && has_nxt) ? b_nxt_v : b_cur_v;
+    // A3 / B3: the free buffer of the three-buffer operand, stage kt + 2's
+    char* const Af = A3 ? abuf3((PHASE + 2) % 3) : Aw;
+    char* const Bf = B3 ? bbuf3b((PHASE + 2) % 3) : Bw;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if (ks == BS) {
         __builtin_amdgcn_sched_barrier(0);
         // stage g + 1 landed; stages g + 2 .. issued - 1 may still be in flight
-        // (epilogue stores issued after them only make this wait longer).  A3:
-        // the last AI instructions (A of step g + 2) may still be in flight.
-        if constexpr (A3)
-          wait_vmcnt<AI>();
-        else if constexpr (B3)
-          wait_vmcnt<BI>();
+        // (epilogue stores issued after them only make this wait longer).  A3 /
+        // B3: this step's early instructions may still be in flight.
+        if constexpr (EARLY)
+          wait_vmcnt<A3 ? AI : BI>();
+        else if constexpr (A3 || B3)
+          wait_vmcnt<0>();
         else
           wait_vmcnt_upto<S - 2, PER>(min(S - 2, max(0, issued - (gstep + 2))));
         __syncthreads();
         if (fill && !fill_cur && ks_fill == nk) {
           // the next tile's perm block went out at this tile's start, before
           // stage kt + 1 when nk >= 2S - 1; otherwise wait for it explicitly.
-          // B3: its VGPR is read after all of this wave's loads landed (this
-          // step's B(g + 2) included), once per tile
-          if (B3 || nk < 2 * S - 1) wait_vmcnt<0>();
+          // B3: this is the LATE step, whose wait above was for every load
+          if (!B3 && nk < 2 * S - 1) wait_vmcnt<0>();
           finish_rows(rows_fill);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -624,30 +619,50 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
           else if (!LAST)
             load_frag(As_n, Bs_n, ks + LA - KS, slot(ks + LA), t);
         }
-        if (ks >= BS) {
+        if constexpr (A3 || B3) {
+          // The three-buffer operand's F3 instructions go out over the substeps
+          // before the barrier (its buffer was free when the step began), the
+          // other operand's over those after it; LATE: both after it.
+          constexpr int F3 = A3 ? AI : BI;
+          constexpr int W0 = BS * NT, W1 = (KS - BS) * NT;
+          auto issue_f3 = [&](int q) __attribute__((always_inline)) {
+            if constexpr (A3)
+              issue_a(Af, a_fill, k0_fill, q);
+            else
+              issue_b(Bf, b_fill, k0_fill, q);
+          };
+          auto issue_f2 = [&](int q) __attribute__((always_inline)) {
+            if constexpr (A3)
+              issue_b(Bw, b_fill, k0_fill, q);
+            else
+              issue_ag(Aw, rows_fill[q < AI ? q : 0], a_fill, k0_fill, q);
+          };
+          if (ks < BS) {
+            if constexpr (EARLY) {
+              const int w = ks * NT + t;
+#pragma unroll
+              for (int q = (w * F3) / W0; q < ((w + 1) * F3) / W0; ++q) issue_f3(q);
+            }
+          } else {
+            const int w = (ks - BS) * NT + t;
+            constexpr int PL = EARLY ? PER - F3 : PER;
+#pragma unroll
+            for (int q = (w * PL) / W1; q < ((w + 1) * PL) / W1; ++q) {
+              if (q < PER - F3)
+                issue_f2(q);
+              else
+                issue_f3(q - (PER - F3));
+            }
+          }
+        } else if (ks >= BS) {
           // DMA instructions q in [w * PER / W, (w + 1) * PER / W) go out after
           // the w-th MFMA since the barrier: the stage's PER instructions
           // spread over the substeps from BS on.
           constexpr int W = (KS - BS) * NT;
           const int w = (ks - BS) * NT + t;
 #pragma unroll
-          for (int q = (w * PER) / W; q < ((w + 1) * PER) / W; ++q) {
-            if constexpr (A3) {
-              // B first: the stage barrier's wait leaves only A in flight
-              if (q < BI)
-                issue_b(Bw, b_fill, k0_fill, q);
-              else if (!LAST)
-                issue_a(Aw, a3_fill, k0_afill, q - BI);
-            } else if constexpr (B3) {
-              // A first: the stage barrier's wait leaves only B in flight
-              if (q < AI)
-                issue_ag(Aw, rows_fill[q < AI ? q : 0], a_fill, k0_fill, q);
-              else if (!LAST)
-                issue_b(Bw, b3_fill, k0_afill, q - AI);
-            } else {
-              issue_one(cb, row_of(rows_fill, q), a_fill, b_fill, k0_fill, q);
-            }
-          }
+          for (int q = (w * PER) / W; q < ((w + 1) * PER) / W; ++q)
+            issue_one(cb, row_of(rows_fill, q), a_fill, b_fill, k0_fill, q);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -664,22 +679,22 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
   using P2 = std::integral_constant<int, 2>;
   for (;;) {
     if constexpr (NSLOT == 2) {
-      kstep(T_{}, F_{}, P0{}, 0);
-      for (int kt = 1; kt + 1 < nk; ++kt) kstep(F_{}, F_{}, P0{}, kt);
-      kstep(F_{}, T_{}, P0{}, nk - 1);
+      kstep(T_{}, F_{}, P0{}, 0, F_{});
+      for (int kt = 1; kt + 1 < nk; ++kt) kstep(F_{}, F_{}, P0{}, kt, F_{});
+      kstep(F_{}, T_{}, P0{}, nk - 1, F_{});
     } else {
       // nk % 3 == 0 and nk >= 6, so every tile starts at gstep % 3 == 0
-      kstep(T_{}, F_{}, P0{}, 0);
-      kstep(F_{}, F_{}, P1{}, 1);
-      kstep(F_{}, F_{}, P2{}, 2);
+      kstep(T_{}, F_{}, P0{}, 0, F_{});
+      kstep(F_{}, F_{}, P1{}, 1, F_{});
+      kstep(F_{}, F_{}, P2{}, 2, F_{});
       for (int kt = 3; kt + 3 < nk; kt += 3) {
-        kstep(F_{}, F_{}, P0{}, kt);
-        kstep(F_{}, F_{}, P1{}, kt + 1);
-        kstep(F_{}, F_{}, P2{}, kt + 2);
+        kstep(F_{}, F_{}, P0{}, kt, F_{});
+        kstep(F_{}, F_{}, P1{}, kt + 1, F_{});
+        kstep(F_{}, F_{}, P2{}, kt + 2, F_{});
       }
-      kstep(F_{}, F_{}, P0{}, nk - 3);
-      kstep(F_{}, F_{}, P1{}, nk - 2);
-      kstep(F_{}, T_{}, P2{}, nk - 1);
+      kstep(F_{}, F_{}, P0{}, nk - 3, F_{});
+      kstep(F_{}, F_{}, P1{}, nk - 2, std::bool_constant<B3>{});
+      kstep(F_{}, T_{}, P2{}, nk - 1, F_{});
     }
 
     if constexpr (MODE == 5) {
@@ -1130,19 +1145,6 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
       dma_rows(nxt);
       a_nxt = a_base_of(nxt);
       b_nxt = b_base_of(nxt);
-    }
-    if constexpr (A3) {
-      // the new tile's third A stage, into the epilogue region: this wave's
-      // slice is its own region, whose epilogue LDS reads completed before
-      // their global stores, and every wave's last reads of it as the old
-      // tile's A buffer preceded the last step's stage barrier
-#pragma unroll
-      for (int q = 0; q < AI; ++q) issue_a(epi_base, a_cur, 2 * BK, q);
-    }
-    if constexpr (B3) {
-      // the same for the new tile's third B stage
-#pragma unroll
-      for (int j = 0; j < BI; ++j) issue_b(epi_base, b_cur, 2 * BK, j);
     }
     // first substeps' fragments of the new tile (its stage 0 landed at the
     // last stage barrier)
