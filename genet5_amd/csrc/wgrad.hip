@@ -18,8 +18,10 @@
 // The structure is the grouped GEMMs' (grouped_gemm.hip): a persistent grid of
 // one workgroup per CU, 256 x 256 tiles, 4 waves in a 2 x 2 grid with 128 x 128
 // fp32 accumulators each in AGPRs, two 64 KB LDS stages filled by
-// global_load_lds_dwordx4, three fragment register slots, each stage's refill
-// spread over the MFMAs, and an LDS-staged epilogue.  What differs is the
+// global_load_lds_dwordx4, a third A buffer in the epilogue region, three
+// fragment register slots, each stage's refill spread over all MFMAs of a k-step
+// (A's over its first half, into the free third buffer, B's over its second),
+// and an LDS-staged epilogue.  What differs is the
 // operand layout: the reduction dimension (tokens) is the outer one in memory,
 // so a stage holds 64 token rows of 512 bytes per operand, and an MFMA operand
 // (8 consecutive tokens of one feature per lane) comes from two
@@ -193,15 +195,15 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
     lds_dma16_s(src, uint32_t(half * ld2) + chunk_off[q & 1],
                 lds_of(dst + (wave * kAI + q) * 1024));
   };
-  // DMA instruction q (q < kAI: A slot q, else B slot q - kAI) of the stage at
-  // token k0 of the tile with DMA bases a, b into buffer buf.
-  auto issue_one = [&](int buf, const char* a, int lda2, const char* b, int ldb2, int k0, int q)
-      __attribute__((always_inline)) {
-    char* As = smem + buf * kStage;
-    if (q < kAI)
-      issue(As, a, lda2, k0, q);
-    else
-      issue(As + kOpBytes, b, ldb2, k0, q - kAI);
+  // A buffer of k-step phase p (k-step mod 3): buffer 2 is the epilogue region
+  // (one A operand; wave w's DMA slice of it is wave w's own region).  Tiles
+  // start at phase 0, so a tile's last step reads buffer 2 and the next tile's
+  // first step refills it after the epilogue.  B buffer of k-step g: g % 2.
+  auto abuf = [&](int p) __attribute__((always_inline)) -> char* {
+    return smem + (p == 2 ? 2 * kStage : p * kStage);
+  };
+  auto bbuf = [&](int g) __attribute__((always_inline)) -> char* {
+    return smem + (g & 1) * kStage + kOpBytes;
   };
 
   // Transposing fragment reads.  For fragment f of a 128-feature wave block at
@@ -236,18 +238,18 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
 
   bf16x8 mfr[3][kMB], nfr[3][kNB];
   // fragment f < kMB: C-row (A) block f; else C-column (B) block f - kMB
-  auto load_frag = [&](int buf, int ks, int slot_, int f) __attribute__((always_inline)) {
-    const uint32_t base = smem_lds + uint32_t(buf * kStage);
+  auto load_frag = [&](const char* As, const char* Bs, int ks, int slot_, int f)
+      __attribute__((always_inline)) {
     if (f < kMB)
-      mfr[slot_][f] = frag_at(base, fA0, fA1, ks, f);
+      mfr[slot_][f] = frag_at(lds_of(As), fA0, fA1, ks, f);
     else
-      nfr[slot_][f - kMB] = frag_at(base + kOpBytes, fB0, fB1, ks, f - kMB);
+      nfr[slot_][f - kMB] = frag_at(lds_of(Bs), fB0, fB1, ks, f - kMB);
   };
-  auto load_first_frags = [&](int buf) __attribute__((always_inline)) {
+  auto load_first_frags = [&](const char* As, const char* Bs) __attribute__((always_inline)) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int f = 0; f < kMB + kNB; ++f) load_frag(buf, ks, ks, f);
+      for (int f = 0; f < kMB + kNB; ++f) load_frag(As, Bs, ks, ks, f);
   };
 
   WTile cur, nxt;
@@ -264,14 +266,17 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
   const f32x16 zero16 = {};
 
 #pragma unroll
-  for (int st = 0; st < 2; ++st)
+  for (int st = 0; st < 2; ++st) {
 #pragma unroll
-    for (int q = 0; q < kPER; ++q) issue_one(st, cur.a, cur.lda2, cur.b, cur.ldb2, st * kBK, q);
+    for (int q = 0; q < kAI; ++q) issue(abuf(st), cur.a, cur.lda2, st * kBK, q);
+#pragma unroll
+    for (int q = 0; q < kAI; ++q) issue(bbuf(st), cur.b, cur.ldb2, st * kBK, q);
+  }
   wait_vmcnt<kPER>();  // stage 0 landed
   __syncthreads();
-  load_first_frags(0);
+  load_first_frags(abuf(0), bbuf(0));
 
-  int gstep = 0;  // k-step counter over the workgroup's tiles; buffer = gstep % 2
+  int gstep = 0;  // k-step counter over the workgroup's tiles; B buffer = gstep % 2
   const int tok_l = lane & 31;
 
   auto kstep = [&](auto first_c, auto last_c, auto phase_c, int kt)
@@ -280,11 +285,14 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
     constexpr bool LAST = decltype(last_c)::value;
     constexpr int PHASE = decltype(phase_c)::value;
     auto slot = [](int ks) { return (PHASE * kKS + ks) % 3; };
-    const int cb = gstep & 1;
-    const int nb = cb ^ 1;
-    // the stage that refills buffer cb: k-step kt + 2 of this tile or of the
-    // next (past the end of the tile list: stage 0 of this tile again, into a
-    // buffer no later step reads)
+    char* const As = abuf(PHASE);
+    char* const Bs = bbuf(gstep);
+    char* const As_n = abuf((PHASE + 1) % 3);
+    char* const Bs_n = bbuf(gstep + 1);
+    char* const Af = abuf((PHASE + 2) % 3);  // free since the previous step's barrier
+    // the stage these refills load: k-step kt + 2 of this tile or of the next
+    // (past the end of the tile list: stage 0 of this tile again, into a buffer
+    // no later step reads)
     const int ks_fill = kt + 2;
     const bool fill_cur = ks_fill < cur.nk;
     const bool use_nxt = !fill_cur && has_nxt;
@@ -304,8 +312,8 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
     for (int ks = 0; ks < kKS; ++ks) {
       if (ks == 2) {
         __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt<0>();  // stage g + 1 landed
-        __syncthreads();  // and every wave is done reading buffer cb
+        wait_vmcnt<kAI>();  // stage g + 1 landed (A of g + 2 may be in flight)
+        __syncthreads();    // and every wave is done reading this step's buffers
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -320,17 +328,22 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
                                                               acc[i][j], 0, 0, 0);
         if (t < kMB + kNB) {
           if (ks + 2 < kKS)
-            load_frag(cb, ks + 2, slot(ks + 2), t);
+            load_frag(As, Bs, ks + 2, slot(ks + 2), t);
           else if (!LAST)
-            load_frag(nb, ks + 2 - kKS, slot(ks + 2), t);
+            load_frag(As_n, Bs_n, ks + 2 - kKS, slot(ks + 2), t);
         }
-        if (ks >= 2) {
-          // one DMA instruction after every other MFMA of the last two substeps
+        {
+          // one DMA instruction after every fourth MFMA: A's over the first two
+          // substeps, B's over the last two
           constexpr int W = 2 * kNT;
-          const int w = (ks - 2) * kNT + t;
+          const int w = (ks & 1) * kNT + t;
 #pragma unroll
-          for (int q = (w * kPER) / W; q < ((w + 1) * kPER) / W; ++q)
-            issue_one(cb, fa, fla, fb, flb, k0_fill, q);
+          for (int q = (w * kAI) / W; q < ((w + 1) * kAI) / W; ++q) {
+            if (ks < 2)
+              issue(Af, fa, fla, k0_fill, q);
+            else
+              issue(Bs, fb, flb, k0_fill, q);
+          }
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -409,7 +422,7 @@ __global__ __launch_bounds__(256) void wgrad_persist_kernel(WgradArgs args) {
     if (has_nxt) wgrad_decode(args, off, lo + slot + (ui + 1) * nslot, wave, nxt);
     // first substeps' fragments of the new tile (its stage 0 landed at the
     // last stage barrier)
-    load_first_frags(gstep & 1);
+    load_first_frags(abuf(0), bbuf(gstep));
   }
 }
 
