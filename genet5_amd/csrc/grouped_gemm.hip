@@ -45,6 +45,7 @@
 // feature blocks 2j and 2j+1 hold gate and up of the same 32 h columns in the
 // same lanes; silu(g) * u is formed in registers and only h is stored (bf16).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "gemm_common.h"
@@ -214,17 +215,10 @@ struct Units {
   int first, stride, count, base;
 };
 
-// Bytes of a wave's epilogue region: 8 KB, or 4 KB in the 128 x 128 tiles,
-// whose workgroups run two per CU (2 x 80 KB of LDS).
-template <int BM, int BN>
-constexpr int epi_bytes() {
-  return BM == 128 && BN == 128 ? 4096 : kEpiBytesPerWave;
-}
-
 // LDS bytes of the persistent kernel for a BM x BN tile (stages + epilogue).
 template <int BM, int BN, int BK, int S>
 constexpr int persist_smem_bytes() {
-  return S * (BM + BN) * BK * 2 + 4 * epi_bytes<BM, BN>();
+  return S * (BM + BN) * BK * 2 + 4 * kEpiBytesPerWave;
 }
 
 // One pass of the persistent tile loop over the units `un` (BN = BNF for full
@@ -265,7 +259,7 @@ __device__ __forceinline__ void tile_loop(const GemmArgs& args, const Offsets& o
   static_assert(NSLOT == 2 || (NSLOT == 3 && KS == 4), "fragment slots");
   static_assert(BK == 32 || BK == 64, "BK");
   static_assert(HALF ? 2 * BN == BNF : BN == BNF, "tile width");
-  constexpr int EPI = epi_bytes<BM, BNF>();  // the wave's epilogue region
+  constexpr int EPI = kEpiBytesPerWave;  // the wave's epilogue region
   static_assert(S >= 2 && S * STAGE + 4 * EPI <= 160 * 1024, "LDS");
   static_assert((S - 2) * PER < 64, "vmcnt range");
   constexpr bool SWIGLU = MODE == 1 || MODE == 3 || MODE == 5;
@@ -1238,16 +1232,190 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
   }
 }
 
-// Two workgroups per CU (two waves per SIMD, 256 registers per lane, at most 80
-// KB of LDS each): twice the operand bytes in flight per CU, for launches with
-// about one tile per CU, whose k-loops wait on load latency.
-template <int BM, int BN, int BK, int S, int NSLOT, int GM, int MODE, bool HALF_TAIL,
-          bool DROP = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-grouped_gemm_persist2_kernel(GemmArgs args) {
-  static_assert(persist_smem_bytes<BM, BN, BK, S>() <= 80 * 1024, "two workgroups per CU");
-  __shared__ __attribute__((aligned(1024))) char smem[persist_smem_bytes<BM, BN, BK, S>()];
-  persist_body<BM, BN, BK, S, NSLOT, GM, MODE, HALF_TAIL, DROP, false>(args, smem);
+// ---------------------------------------------------------------------------
+// Ring kernel: the in-place products with few rows (small_m in the launchers: a
+// short sequence, a shard's share, a one-expert projection of one window).
+//
+// With less than about one and a half 256 x 256 tiles per CU the persistent
+// kernel's workgroups each run one long tile: its k-loop waits for the two
+// stages in flight, most CUs idle, and a partial tile computes its padding rows.
+// Here a tile is up to MAXMB 32-row blocks of one expert, exactly as many as it
+// has rows for (the expert's blocks are dealt evenly to its tiles), by 128
+// columns; the four waves take 32 columns each and share the rows.  One
+// workgroup per tile, one (OCC = 1) or two (OCC = 2) to a CU; all of its LDS is a
+// ring of k-stages (MB = 1: 20 KB each), so up to seven are in flight; fragments
+// are read one 16-k substep ahead.  The weight stream (each weight row read once
+// per m-tile, from beyond the L2) bounds MB = 1, the LDS fragment reads
+// (MB + 1 per MB MFMAs and wave) MB = 4: about 0.25 + 0.1 MB us a k-step.
+// Every accumulator takes its k in the persistent kernel's order, so the outputs
+// are the same bit for bit.
+//
+// Measured against the 128 x 128 (two workgroups per CU) and 128 x 256 persistent
+// tiles that served these launches before (one GPU, captured loops, 16 experts):
+//   h . Wd^T, K = 3,072, N = 768:  96 rows 45 -> 18 us, 1,554 45 -> 21,
+//     4,096 45 -> 31-33, 9,100 51 -> 49, 18,000 95 -> 94;
+//   dGU . Wgu, K = 6,144, N = 768: 512 rows 83 -> 32, 2,200 84 -> 48,
+//     9,100 117 -> 104, 18,000 239 -> 209;
+//   one expert, K = 768: 512 x 2,304 11.9 -> 7.4, 2,048 x 2,304 13.4 -> 11.9,
+//     4,550 x 2,304 25.8 -> 23.7.
+struct RingTile {
+  int e, p_begin, p_end, a_row, n0, mb;  // mb: 32-row blocks of the tile
+};
+
+// Tile u of the launch: expert-major, inside an expert in groups of four m-tiles
+// swept across the n-tiles, as decode_tile_u.
+template <int MAXMB, bool PADA>
+__device__ __forceinline__ void ring_decode(const GemmArgs& args, const Offsets& off, int u,
+                                            int ntn, int bn, RingTile& t) {
+  int e = 0, nb = 0, mt = 0;
+  for (; e < args.n_experts; ++e) {
+    nb = (expert_rows(args, off, e) + 31) / 32;
+    mt = (nb + MAXMB - 1) / MAXMB;
+    if (u < mt * ntn) break;
+    u -= mt * ntn;
+  }
+  constexpr int GM = 4;
+  const int g = u / (GM * ntn);
+  const int first_m = g * GM;
+  const int gs = min(GM, mt - first_m);
+  const int rr = u - g * GM * ntn;
+  const int m = first_m + rr % gs;
+  const int q = nb / mt, r = nb % mt;
+  t.e = e;
+  t.mb = q + (m < r ? 1 : 0);
+  const int row0 = 32 * (m * q + min(m, r));
+  t.p_begin = off(e) + row0;
+  t.p_end = off(e) + expert_rows(args, off, e);
+  t.a_row = (PADA ? pad_start(args, off, e) : off(e)) + row0;
+  t.n0 = (rr / gs) * bn;
+}
+
+// One tile of MB 32-row blocks.  S stages of the ring fit SMEM bytes of LDS.
+template <int MB, int NB, int SMEM, bool PADA>
+__device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& tc, char* smem) {
+  constexpr int BK = 64, RB = BK * 2, KS = BK / 16;
+  constexpr int BN = 128 * NB;
+  constexpr int AI = MB, BI = 4 * NB, PER = AI + BI;  // DMA instructions per wave and stage
+  constexpr int A_BYTES = MB * 4096, STAGE = A_BYTES + BN * RB;
+  constexpr int S = SMEM / STAGE < 8 ? SMEM / STAGE : 8;
+  static_assert(S >= 2 && (S - 1) * PER < 64, "stages");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K = args.K, nk = K / BK;
+  const uint32_t smem_lds = lds_addr(smem);
+  // DMA instruction q of a wave fills the 8 rows of block 4 q + wave of an operand
+  // (chunk c of row r at c ^ ((r >> 1) & 7), as the persistent kernel's stages).
+  // A rows past the expert's end are the next expert's or the buffer's padding
+  // rows (at most 31 past the last), computed and never stored.
+  const int lrow = lane >> 3;
+  const uint32_t voff =
+      uint32_t(lrow * K * 2 + (((lane & 7) ^ (((wave & 1) * 4 + (lrow >> 1)) & 7)) * 16));
+  const uint32_t blk_bytes = uint32_t(32 * K * 2);  // 4 blocks of 8 rows
+  const char* a_base =
+      reinterpret_cast<const char*>(args.A + (int64_t(tc.a_row) + wave * 8) * K);
+  const char* b_base =
+      reinterpret_cast<const char*>(args.B + (int64_t(tc.e) * args.Nout + tc.n0 + wave * 8) * K);
+  auto issue = [&](int st, int buf) __attribute__((always_inline)) {
+    const uint32_t dst = smem_lds + uint32_t(buf) * STAGE + uint32_t(wave) * 1024;
+    const int k0 = st * RB;
+#pragma unroll
+    for (int q = 0; q < BI; ++q)
+      lds_dma16_s(b_base + k0 + size_t(q) * blk_bytes, voff, dst + A_BYTES + q * 4096);
+#pragma unroll
+    for (int q = 0; q < AI; ++q)
+      lds_dma16_s(a_base + k0 + size_t(q) * blk_bytes, voff, dst + q * 4096);
+  };
+#pragma unroll
+  for (int st = 0; st < S; ++st)
+    if (st < nk) issue(st, st);
+
+  f32x16 acc[NB][MB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) acc[i][j] = f32x16{};
+  const int a_row = (lane & 31) * RB;
+  const int b_row = (wave * NB * 32 + (lane & 31)) * RB + A_BYTES;
+  const int khalf = lane >> 5;
+  const int rsw = ((lane & 31) >> 1) & 7;
+  bf16x8 af[2][MB], bfr[2][NB];
+  auto frags = [&](int buf, int ks, int sl) __attribute__((always_inline)) {
+    const char* st = smem + buf * STAGE;
+    const int pc = ((ks * 2 + khalf) ^ rsw) * 16;
+#pragma unroll
+    for (int f = 0; f < NB; ++f)
+      bfr[sl][f] = *reinterpret_cast<const bf16x8*>(st + b_row + f * 32 * RB + pc);
+#pragma unroll
+    for (int f = 0; f < MB; ++f)
+      af[sl][f] = *reinterpret_cast<const bf16x8*>(st + a_row + f * 32 * RB + pc);
+  };
+  wait_vmcnt_upto<S - 1, PER>(min(S - 1, nk - 1));
+  __syncthreads();
+  frags(0, 0, 0);
+  int buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    const int nbuf = buf + 1 == S ? 0 : buf + 1;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks < KS - 1) {
+        frags(buf, ks + 1, (ks + 1) & 1);
+      } else {
+        // stage kt + 1 landed, and every wave has read its last fragments of
+        // this stage: its buffer takes stage kt + S
+        wait_vmcnt_upto<S - 2, PER>(max(0, min(S - 2, nk - 2 - kt)));
+        __syncthreads();
+        if (kt + 1 < nk) frags(nbuf, 0, 0);
+        if (kt + S < nk) issue(kt + S, buf);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks & 1][i], af[ks & 1][j],
+                                                              acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    buf = nbuf;
+  }
+  // (the last barrier came after every wave's last LDS reads)
+  constexpr int RBY = NB * 64, CR = RBY / 16, LPR = 256 / RBY;
+  char* epi = smem + wave * 32 * MB * RBY;
+#pragma unroll
+  for (int j = 0; j < MB; ++j) {
+    const int row = j * 32 + (lane & 31);
+    const int swz = (row / LPR) % CR;
+#pragma unroll
+    for (int ob = 0; ob < NB; ++ob)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<uint2*>(epi + row * RBY + (((ob * 4 + q) ^ swz) * 16) + khalf * 8) =
+            make_uint2(pack_bf16x2(acc[ob][j][4 * q], acc[ob][j][4 * q + 1]),
+                       pack_bf16x2(acc[ob][j][4 * q + 2], acc[ob][j][4 * q + 3]));
+  }
+  store_pass<32 * MB, RBY>(epi, args.C + tc.n0 + wave * NB * 32, args.ldc, tc.p_begin, tc.p_end,
+                           lane);
+}
+
+template <int MAXMB, int NB, int OCC, bool PADA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void
+grouped_gemm_ring_kernel(GemmArgs args) {
+  constexpr int SMEM = 160 * 1024 / OCC;
+  __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+  constexpr int BN = 128 * NB;
+  const Offsets off = load_offsets(args.offsets, args.n_experts);
+  const int ntn = args.Nout / BN;
+  int total = 0;
+  for (int e = 0; e < args.n_experts; ++e)
+    total += (((expert_rows(args, off, e) + 31) / 32 + MAXMB - 1) / MAXMB) * ntn;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
+  if (lo + slot >= hi) return;
+  RingTile tc;
+  ring_decode<MAXMB, PADA>(args, off, lo + slot, ntn, BN, tc);
+  if (tc.mb == 1) ring_tile<1, NB, SMEM, PADA>(args, tc, smem);
+  if constexpr (MAXMB >= 2) if (tc.mb == 2) ring_tile<2, NB, SMEM, PADA>(args, tc, smem);
+  if constexpr (MAXMB >= 3) if (tc.mb == 3) ring_tile<3, NB, SMEM, PADA>(args, tc, smem);
+  if constexpr (MAXMB >= 4) if (tc.mb == 4) ring_tile<4, NB, SMEM, PADA>(args, tc, smem);
 }
 
 }  // namespace
@@ -1338,26 +1506,6 @@ __global__ void cast_f32_bf16_kernel(const float* __restrict__ x, uint16_t* __re
 #ifndef G5_DN_GM
 #define G5_DN_GM 4
 #endif
-
-// Small-M down products on 128 x 128 tiles, two workgroups per CU (0: one
-// 128 x 256 workgroup per CU).
-#ifndef G5_SMALLM_TWO_PER_CU
-#define G5_SMALLM_TWO_PER_CU 1
-#endif
-
-// The two-per-CU kernel (grid up to twice the CU count).
-template <int BM, int BN, int BK, int S, int GM, int MODE, bool HALF_TAIL, bool DROP = false>
-void launch_persist2(unsigned grid, const GemmArgs& a, hipStream_t st) {
-  const int nk = a.K / BK;
-  if (nk % 3 == 0 && nk >= 6)
-    hipLaunchKernelGGL(
-        (grouped_gemm_persist2_kernel<BM, BN, BK, S, 3, GM, MODE, HALF_TAIL, DROP>),
-        dim3(grid), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL(
-        (grouped_gemm_persist2_kernel<BM, BN, BK, S, 2, GM, MODE, HALF_TAIL, DROP>),
-        dim3(grid), dim3(256), 0, st, a);
-}
 
 // Persistent launch: three fragment slots when the k-step count allows it.
 // PADA: A rows in a per-expert padded layout (a.a_rows_per_expert != 0).
@@ -1517,14 +1665,76 @@ hipError_t launch_dh_swiglu(const uint16_t* dy_pad, int kmax, const int32_t* off
   return hipGetLastError();
 }
 
-// Small M (a shard's share of the tokens: one wave of 256-row tiles or less for
-// the CUs): 128-row m-tiles, twice the tiles at half the work each, and less
-// padding past each expert's last row.  The row count is the host's N * k (the
-// per-expert counts stay on the device), so the test is on the full-tile count
-// the rows would give if packed.
+namespace {
+
+// Small M: fewer rows than one and a half 256 x 256 tiles per CU would take if
+// packed (the per-expert counts stay on the device).
 inline bool small_m(int64_t rows, int nout, unsigned ncu) {
-  return (rows / 256) * (nout / 256) < int64_t(3 * ncu / 2);
+  return rows * nout < int64_t(3 * ncu / 2) * 256 * 256;
 }
+
+template <int MAXMB, int OCC, bool PADA>
+void launch_ring_tiles(const GemmArgs& a, int64_t rows, hipStream_t st) {
+  // tiles: sum_e ceil(ceil(cnt_e / 32) / MAXMB) <= rows / (32 MAXMB) + E per column
+  const int64_t mt = (rows + 32 * MAXMB - 1) / (32 * MAXMB) + a.n_experts;
+  const unsigned grid = unsigned((mt * (a.Nout / 128) + 7) / 8 * 8);
+  hipLaunchKernelGGL((grouped_gemm_ring_kernel<MAXMB, 1, OCC, PADA>), dim3(grid), dim3(256), 0,
+                     st, a);
+}
+
+// The ring kernel's tile height: the smallest whose tiles (for experts of the
+// mean row count and two standard deviations of uniform routing more) do not
+// outnumber the CUs, else the smallest with at most two per CU, else 128 rows.
+// Fewer rows per tile keep more CUs pulling the weight stream; a tile more than
+// the resident workgroups costs a whole tile's time (down, 4,096 rows: 432
+// 64-row tiles 33 us, 288 96-row ones 41).  128- and 96-row tiles with at most
+// one per CU take all of its LDS (OCC = 1: 26.6 against 33.5 us at 1,554 rows,
+// 96-row tiles; two stages of half the LDS leave one in flight), smaller ones
+// start sooner with half (one expert, 300 x 768 x 768: 6.2 against 6.9 us).
+template <bool PADA>
+void launch_ring(const GemmArgs& a, int64_t rows, unsigned ncu, hipStream_t st) {
+  const double mean = double(rows) / a.n_experts;
+  const int64_t m = int64_t(mean + (a.n_experts > 1 ? 2.0 * std::sqrt(mean) : 0.0));
+  const int64_t nb = std::max<int64_t>(1, (m + 31) / 32);
+  auto tiles = [&](int mb) { return (nb + mb - 1) / mb * a.n_experts * (a.Nout / 128); };
+  int mb = 1, per_cu = 1;
+  while (mb < 4 && tiles(mb) > int64_t(ncu)) ++mb;
+  if (tiles(mb) > int64_t(ncu)) {
+    per_cu = 2;
+    for (mb = 1; mb < 4 && tiles(mb) > 2 * int64_t(ncu);) ++mb;
+  }
+  if (mb == 1)
+    launch_ring_tiles<1, 2, PADA>(a, rows, st);
+  else if (mb == 2)
+    launch_ring_tiles<2, 2, PADA>(a, rows, st);
+  else if (mb == 3 && per_cu == 1)
+    launch_ring_tiles<3, 1, PADA>(a, rows, st);
+  else if (mb == 3)
+    launch_ring_tiles<3, 2, PADA>(a, rows, st);
+  else if (per_cu == 1)
+    launch_ring_tiles<4, 1, PADA>(a, rows, st);
+  else
+    launch_ring_tiles<4, 2, PADA>(a, rows, st);
+}
+
+// The MODE 0 products (A rows in place, or per-expert padded with PADA).
+template <bool PADA>
+hipError_t launch_in_place(const GemmArgs& a, int64_t rows, hipStream_t st) {
+  const unsigned ncu = unsigned(device_cu_count());
+  if (small_m(rows, a.Nout, ncu)) {
+    launch_ring<PADA>(a, rows, ncu, st);
+  } else if (a.Nout % 256 == 0) {
+    const unsigned grid = std::min(grid_bound<256, 256>(rows, a.n_experts, a.Nout), ncu);
+    launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, true, false, PADA>(grid, a, st);
+  } else {
+    const unsigned grid = std::min(grid_bound<256, 128>(rows, a.n_experts, a.Nout), ncu);
+    launch_persist<256, 128, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false, false, PADA>(grid, a,
+                                                                                      st);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace
 
 hipError_t launch_down(const uint16_t* h, const int32_t* offsets, const uint16_t* wd,
                        uint16_t* y_perm, const g5moe_shape& s, hipStream_t st) {
@@ -1542,21 +1752,7 @@ hipError_t launch_down(const uint16_t* h, const int32_t* offsets, const uint16_t
   a.Nout = s.d_model;
   a.ldc = s.d_model;
   if (a.K < G5_DN_STAGES * G5_DN_BK) return hipErrorInvalidValue;
-  const unsigned ncu = unsigned(device_cu_count());
-  if (G5_SMALLM_TWO_PER_CU && a.Nout % 256 == 0 && small_m(nk, a.Nout, ncu)) {
-    const unsigned grid = std::min(grid_bound<128, 128>(nk, s.n_experts, a.Nout), 2 * ncu);
-    launch_persist2<128, 128, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false>(grid, a, st);
-  } else if (a.Nout % 256 == 0 && small_m(nk, a.Nout, ncu)) {
-    const unsigned grid = std::min(grid_bound<128, 256>(nk, s.n_experts, a.Nout), ncu);
-    launch_persist<128, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false>(grid, a, st);
-  } else if (a.Nout % 256 == 0) {
-    const unsigned grid = std::min(grid_bound<256, 256>(nk, s.n_experts, a.Nout), ncu);
-    launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, true>(grid, a, st);
-  } else {
-    const unsigned grid = std::min(grid_bound<256, 128>(nk, s.n_experts, a.Nout), ncu);
-    launch_persist<256, 128, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false>(grid, a, st);
-  }
-  return hipGetLastError();
+  return launch_in_place<false>(a, nk, st);
 }
 
 hipError_t launch_gate_up_raw(const uint16_t* xb, const int32_t* perm, const int32_t* offsets,
@@ -1600,34 +1796,8 @@ hipError_t launch_grouped_nt(const uint16_t* A, const int32_t* offsets, const ui
   a.K = K;
   a.Nout = Nout;
   a.ldc = Nout;
-  const unsigned ncu = unsigned(device_cu_count());
-  if (a_rows_per_expert != 0) {  // A rows in a per-expert padded layout
-    if (Nout % 256 == 0 && small_m(rows, Nout, ncu)) {
-      const unsigned grid = std::min(grid_bound<128, 256>(rows, n_experts, Nout), ncu);
-      launch_persist<128, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false, false, true>(grid, a,
-                                                                                        st);
-    } else if (Nout % 256 == 0) {
-      const unsigned grid = std::min(grid_bound<256, 256>(rows, n_experts, Nout), ncu);
-      launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, true, false, true>(grid, a,
-                                                                                       st);
-    } else {
-      const unsigned grid = std::min(grid_bound<256, 128>(rows, n_experts, Nout), ncu);
-      launch_persist<256, 128, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false, false, true>(grid, a,
-                                                                                        st);
-    }
-    return hipGetLastError();
-  }
-  if (Nout % 256 == 0 && small_m(rows, Nout, ncu)) {
-    const unsigned grid = std::min(grid_bound<128, 256>(rows, n_experts, Nout), ncu);
-    launch_persist<128, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false>(grid, a, st);
-  } else if (Nout % 256 == 0) {
-    const unsigned grid = std::min(grid_bound<256, 256>(rows, n_experts, Nout), ncu);
-    launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, true>(grid, a, st);
-  } else {
-    const unsigned grid = std::min(grid_bound<256, 128>(rows, n_experts, Nout), ncu);
-    launch_persist<256, 128, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, false>(grid, a, st);
-  }
-  return hipGetLastError();
+  return a_rows_per_expert != 0 ? launch_in_place<true>(a, rows, st)
+                                : launch_in_place<false>(a, rows, st);
 }
 
 hipError_t launch_pack_gate_up(const uint16_t* wg, const uint16_t* wu, uint16_t* wgu,
