@@ -1233,15 +1233,18 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
 }
 
 // ---------------------------------------------------------------------------
-// Ring kernel: the in-place products with few rows (small_m in the launchers: a
-// short sequence, a shard's share, a one-expert projection of one window).
+// Ring kernel: the products with few rows (the in-place ones under small_m in the
+// launchers: a short sequence, a shard's share, a one-expert projection of one
+// window; the gate|up and dh products of a short sequence, ring_wide).
 //
 // With less than about one and a half 256 x 256 tiles per CU the persistent
 // kernel's workgroups each run one long tile: its k-loop waits for the two
 // stages in flight, most CUs idle, and a partial tile computes its padding rows.
 // Here a tile is up to MAXMB 32-row blocks of one expert, exactly as many as it
 // has rows for (the expert's blocks are dealt evenly to its tiles), by 128
-// columns; the four waves take 32 columns each and share the rows.  One
+// columns; the four waves take 32 columns each (for the SwiGLU modes 16 gate
+// columns and their 16 up columns, so that the pair meets in one lane) and share
+// the rows.  One
 // workgroup per tile, one (OCC = 1) or two (OCC = 2) to a CU; all of its LDS is a
 // ring of k-stages (MB = 1: 20 KB each), so up to seven are in flight; fragments
 // are read one 16-k substep ahead.  The weight stream (each weight row read once
@@ -1258,44 +1261,78 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
 //     9,100 117 -> 104, 18,000 239 -> 209;
 //   one expert, K = 768: 512 x 2,304 11.9 -> 7.4, 2,048 x 2,304 13.4 -> 11.9,
 //     4,550 x 2,304 25.8 -> 23.7.
+// The gate|up and dh figures are at ring_wide.
 struct RingTile {
-  int e, p_begin, p_end, a_row, n0, mb;  // mb: 32-row blocks of the tile
+  int e, p_begin, p_end, a_row, n0;
+  int mb;  // 32-row blocks of the tile; MODE 4: 0 for a tile of zero rows only
 };
 
+// m-tiles of MODE 4's zero rows: 256 rows each.
+constexpr int kRingZeroBlocks = 8;
+
+// Expert e's 32-row blocks with rows, m-tiles of those, and (MODE 4) m-tiles of
+// the rows after them that the weight gradient reads as zeros.
+template <int MAXMB, int MODE>
+__device__ __forceinline__ void ring_blocks(const GemmArgs& args, const Offsets& off, int e,
+                                            int& nb, int& mt, int& zt) {
+  nb = (expert_rows(args, off, e) + 31) / 32;
+  mt = (nb + MAXMB - 1) / MAXMB;
+  zt = 0;
+  if constexpr (MODE == 4)
+    zt = (expert_rows<true>(args, off, e) / 32 - nb + kRingZeroBlocks - 1) / kRingZeroBlocks;
+}
+
 // Tile u of the launch: expert-major, inside an expert in groups of four m-tiles
-// swept across the n-tiles, as decode_tile_u.
-template <int MAXMB, bool PADA>
+// swept across the n-tiles (as decode_tile_u), then its zero tiles.
+template <int MAXMB, int MODE, bool PADA>
 __device__ __forceinline__ void ring_decode(const GemmArgs& args, const Offsets& off, int u,
-                                            int ntn, int bn, RingTile& t) {
-  int e = 0, nb = 0, mt = 0;
+                                            int ntn, RingTile& t) {
+  int e = 0, nb = 0, mt = 0, zt = 0;
   for (; e < args.n_experts; ++e) {
-    nb = (expert_rows(args, off, e) + 31) / 32;
-    mt = (nb + MAXMB - 1) / MAXMB;
-    if (u < mt * ntn) break;
-    u -= mt * ntn;
+    ring_blocks<MAXMB, MODE>(args, off, e, nb, mt, zt);
+    if (u < (mt + zt) * ntn) break;
+    u -= (mt + zt) * ntn;
   }
-  constexpr int GM = 4;
-  const int g = u / (GM * ntn);
-  const int first_m = g * GM;
-  const int gs = min(GM, mt - first_m);
-  const int rr = u - g * GM * ntn;
-  const int m = first_m + rr % gs;
-  const int q = nb / mt, r = nb % mt;
   t.e = e;
-  t.mb = q + (m < r ? 1 : 0);
-  const int row0 = 32 * (m * q + min(m, r));
+  int row0;
+  if (MODE == 4 && u >= mt * ntn) {
+    u -= mt * ntn;
+    t.mb = 0;
+    row0 = 32 * (nb + kRingZeroBlocks * (u / ntn));
+    t.n0 = (u % ntn) * 128;
+  } else {
+    constexpr int GM = 4;
+    const int g = u / (GM * ntn);
+    const int first_m = g * GM;
+    const int gs = min(GM, mt - first_m);
+    const int rr = u - g * GM * ntn;
+    const int m = first_m + rr % gs;
+    const int q = nb / mt, r = nb % mt;
+    t.mb = q + (m < r ? 1 : 0);
+    row0 = 32 * (m * q + min(m, r));
+    t.n0 = (rr / gs) * 128;
+  }
   t.p_begin = off(e) + row0;
-  t.p_end = off(e) + expert_rows(args, off, e);
+  t.p_end = off(e) + expert_rows<MODE == 4>(args, off, e);
   t.a_row = (PADA ? pad_start(args, off, e) : off(e)) + row0;
-  t.n0 = (rr / gs) * bn;
+}
+
+// MODE 4's rows past the expert's last block: zeros in 128 F columns of dGU.
+__device__ __forceinline__ void ring_zero_tile(const GemmArgs& args, const RingTile& tc) {
+  const int rows = min(32 * kRingZeroBlocks, tc.p_end - tc.p_begin);
+  uint16_t* dst = args.C + int64_t(tc.a_row) * args.ldc + 2 * tc.n0;
+  for (int i = threadIdx.x; i < rows * 32; i += 256)  // 32 chunks: 256 packed columns
+    store16_nt(dst + int64_t(i >> 5) * args.ldc + (i & 31) * 8, make_uint4(0, 0, 0, 0));
 }
 
 // One tile of MB 32-row blocks.  S stages of the ring fit SMEM bytes of LDS.
-template <int MB, int NB, int SMEM, bool PADA>
-__device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& tc, char* smem) {
+template <int MB, int SMEM, int MODE, bool DROP, bool PADA>
+__device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& tc,
+                                          const Offsets& off, char* smem) {
   constexpr int BK = 64, RB = BK * 2, KS = BK / 16;
-  constexpr int BN = 128 * NB;
-  constexpr int AI = MB, BI = 4 * NB, PER = AI + BI;  // DMA instructions per wave and stage
+  constexpr int BN = 128;
+  constexpr bool SWIGLU = MODE == 1 || MODE == 5;
+  constexpr int AI = MB, BI = 4, PER = AI + BI;  // DMA instructions per wave and stage
   constexpr int A_BYTES = MB * 4096, STAGE = A_BYTES + BN * RB;
   constexpr int S = SMEM / STAGE < 8 ? SMEM / STAGE : 8;
   static_assert(S >= 2 && (S - 1) * PER < 64, "stages");
@@ -1305,14 +1342,27 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& 
   const uint32_t smem_lds = lds_addr(smem);
   // DMA instruction q of a wave fills the 8 rows of block 4 q + wave of an operand
   // (chunk c of row r at c ^ ((r >> 1) & 7), as the persistent kernel's stages).
-  // A rows past the expert's end are the next expert's or the buffer's padding
-  // rows (at most 31 past the last), computed and never stored.
+  // In-place A rows past the expert's end are the next expert's or the buffer's
+  // padding rows (at most 31 past the last), computed and never stored; gathered
+  // ones repeat the expert's last row.
   const int lrow = lane >> 3;
-  const uint32_t voff =
-      uint32_t(lrow * K * 2 + (((lane & 7) ^ (((wave & 1) * 4 + (lrow >> 1)) & 7)) * 16));
+  const uint32_t chunk = uint32_t(((lane & 7) ^ (((wave & 1) * 4 + (lrow >> 1)) & 7)) * 16);
+  const uint32_t voff = uint32_t(lrow * K * 2) + chunk;
   const uint32_t blk_bytes = uint32_t(32 * K * 2);  // 4 blocks of 8 rows
-  const char* a_base =
-      reinterpret_cast<const char*>(args.A + (int64_t(tc.a_row) + wave * 8) * K);
+  uint32_t aoff[MB];
+  const char* a_base = reinterpret_cast<const char*>(args.A);
+  if constexpr (SWIGLU) {
+    uint32_t v[MB];
+#pragma unroll
+    for (int q = 0; q < MB; ++q)
+      v[q] = uint32_t(args.perm[min(tc.p_begin + q * 32 + wave * 8 + lrow, tc.p_end - 1)]);
+#pragma unroll
+    for (int q = 0; q < MB; ++q) aoff[q] = (v[q] / uint32_t(args.topk)) * uint32_t(K * 2) + chunk;
+  } else {
+    a_base += (int64_t(tc.a_row) + wave * 8) * K * 2;
+#pragma unroll
+    for (int q = 0; q < MB; ++q) aoff[q] = voff + uint32_t(q) * blk_bytes;
+  }
   const char* b_base =
       reinterpret_cast<const char*>(args.B + (int64_t(tc.e) * args.Nout + tc.n0 + wave * 8) * K);
   auto issue = [&](int st, int buf) __attribute__((always_inline)) {
@@ -1322,29 +1372,30 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& 
     for (int q = 0; q < BI; ++q)
       lds_dma16_s(b_base + k0 + size_t(q) * blk_bytes, voff, dst + A_BYTES + q * 4096);
 #pragma unroll
-    for (int q = 0; q < AI; ++q)
-      lds_dma16_s(a_base + k0 + size_t(q) * blk_bytes, voff, dst + q * 4096);
+    for (int q = 0; q < AI; ++q) lds_dma16_s(a_base + k0, aoff[q], dst + q * 4096);
   };
 #pragma unroll
   for (int st = 0; st < S; ++st)
     if (st < nk) issue(st, st);
 
-  f32x16 acc[NB][MB];
+  f32x16 acc[MB];
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int j = 0; j < MB; ++j) acc[i][j] = f32x16{};
-  const int a_row = (lane & 31) * RB;
-  const int b_row = (wave * NB * 32 + (lane & 31)) * RB + A_BYTES;
+  for (int j = 0; j < MB; ++j) acc[j] = f32x16{};
+  // The wave's 32 weight rows: 32 consecutive ones, or (SWIGLU) 16 gate rows and
+  // the 16 up rows they pair with, half of a packed 64-row group; elements 4 q + u
+  // and 8 + 4 q + u (q < 2) of an accumulator are then gate and up of one column.
+  const int r31 = lane & 31;
+  const int b_lrow =
+      SWIGLU ? (wave >> 1) * 64 + (r31 >> 4) * 32 + (wave & 1) * 16 + (r31 & 15) : wave * 32 + r31;
+  const int a_row = r31 * RB;
+  const int b_row = b_lrow * RB + A_BYTES;
   const int khalf = lane >> 5;
-  const int rsw = ((lane & 31) >> 1) & 7;
-  bf16x8 af[2][MB], bfr[2][NB];
+  const int rsw = (r31 >> 1) & 7;  // 16-row offsets leave (row >> 1) & 7 unchanged
+  bf16x8 af[2][MB], bfr[2];
   auto frags = [&](int buf, int ks, int sl) __attribute__((always_inline)) {
     const char* st = smem + buf * STAGE;
     const int pc = ((ks * 2 + khalf) ^ rsw) * 16;
-#pragma unroll
-    for (int f = 0; f < NB; ++f)
-      bfr[sl][f] = *reinterpret_cast<const bf16x8*>(st + b_row + f * 32 * RB + pc);
+    bfr[sl] = *reinterpret_cast<const bf16x8*>(st + b_row + pc);
 #pragma unroll
     for (int f = 0; f < MB; ++f)
       af[sl][f] = *reinterpret_cast<const bf16x8*>(st + a_row + f * 32 * RB + pc);
@@ -1368,54 +1419,192 @@ __device__ __forceinline__ void ring_tile(const GemmArgs& args, const RingTile& 
         if (kt + S < nk) issue(kt + S, buf);
       }
 #pragma unroll
-      for (int i = 0; i < NB; ++i)
-#pragma unroll
-        for (int j = 0; j < MB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks & 1][i], af[ks & 1][j],
-                                                              acc[i][j], 0, 0, 0);
+      for (int j = 0; j < MB; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[ks & 1], af[ks & 1][j], acc[j], 0, 0,
+                                                         0);
       __builtin_amdgcn_sched_barrier(0);
     }
     buf = nbuf;
   }
-  // (the last barrier came after every wave's last LDS reads)
-  constexpr int RBY = NB * 64, CR = RBY / 16, LPR = 256 / RBY;
-  char* epi = smem + wave * 32 * MB * RBY;
+
+  // Epilogue (the last barrier came after every wave's last LDS reads and after
+  // the last stage landed): the workgroup's outputs through LDS to whole row
+  // segments.  256-byte rows (128 columns) keep chunk c of row r at c ^ (r % 16),
+  // 128-byte rows (64 h columns) at c ^ ((r / 2) % 8).
+  char* const t256 = smem;
+  char* const t128 = smem + 32 * MB * 256;
+  auto at256 = [&](int r, int c) __attribute__((always_inline)) -> char* {
+    return t256 + r * 256 + ((c ^ (r & 15)) * 16);
+  };
+  auto at128 = [&](int r, int c) __attribute__((always_inline)) -> char* {
+    return t128 + r * 128 + ((c ^ ((r >> 1) & 7)) * 16);
+  };
+  if constexpr (SWIGLU) {
+    const int hc = (wave >> 1) * 4 + (wave & 1) * 2;   // the wave's first h chunk of the tile
+    const int gc = (wave >> 1) * 8 + (wave & 1) * 2;   // its first gate chunk (up: + 4)
 #pragma unroll
-  for (int j = 0; j < MB; ++j) {
-    const int row = j * 32 + (lane & 31);
-    const int swz = (row / LPR) % CR;
+    for (int j = 0; j < MB; ++j) {
+      const int row = j * 32 + r31;
+      [[maybe_unused]] uint32_t dkey = 0;
+      if constexpr (DROP)
+        dkey = dropout_row_key(uint32_t(args.perm[min(tc.p_begin + row, tc.p_end - 1)]),
+                               args.drop_seed_lo, args.drop_seed_hi);
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob)
+      for (int q = 0; q < 2; ++q) {
+        float hh[4], fa[4], fb[4];
+        [[maybe_unused]] uint32_t rb[4];
+        if constexpr (DROP) {
+          const uint32_t cp = uint32_t(tc.n0 / 2 + (hc + q) * 8 + 4 * khalf) >> 1;
+          const uint32_t b0 = dropout_pair_bits(dkey, cp);
+          const uint32_t b1 = dropout_pair_bits(dkey, cp + 1);
+          rb[0] = b0 & 0xffffu;
+          rb[1] = b0 >> 16;
+          rb[2] = b1 & 0xffffu;
+          rb[3] = b1 >> 16;
+        }
+#pragma unroll
+        for (int uu = 0; uu < 4; ++uu) {
+          const float g = acc[j][4 * q + uu];
+          const float u = acc[j][8 + 4 * q + uu];
+          if constexpr (MODE == 1) {
+            hh[uu] = silu_mul(g, u);
+          } else {
+            // the values of the persistent kernel's MODE 5
+            const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+            const float silu = g * sg;
+            float h = silu * u;
+            float a = u * (sg * (1.0f + g * (1.0f - sg)));
+            float b = silu;
+            if constexpr (DROP) {
+              const bool keep = rb[uu] >= args.drop_thr;
+              h = keep ? h * args.drop_scale : 0.0f;
+              a = keep ? a * args.drop_scale : 0.0f;
+              b = keep ? b * args.drop_scale : 0.0f;
+            }
+            hh[uu] = h;
+            fa[uu] = a;
+            fb[uu] = b;
+          }
+        }
+        *reinterpret_cast<uint2*>(at128(row, hc + q) + khalf * 8) =
+            make_uint2(pack_bf16x2(hh[0], hh[1]), pack_bf16x2(hh[2], hh[3]));
+        if constexpr (MODE == 5) {
+          *reinterpret_cast<uint2*>(at256(row, gc + q) + khalf * 8) =
+              make_uint2(pack_bf16x2(fa[0], fa[1]), pack_bf16x2(fa[2], fa[3]));
+          *reinterpret_cast<uint2*>(at256(row, gc + 4 + q) + khalf * 8) =
+              make_uint2(pack_bf16x2(fb[0], fb[1]), pack_bf16x2(fb[2], fb[3]));
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < MB; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<uint2*>(epi + row * RBY + (((ob * 4 + q) ^ swz) * 16) + khalf * 8) =
-            make_uint2(pack_bf16x2(acc[ob][j][4 * q], acc[ob][j][4 * q + 1]),
-                       pack_bf16x2(acc[ob][j][4 * q + 2], acc[ob][j][4 * q + 3]));
+        *reinterpret_cast<uint2*>(at256(j * 32 + r31, wave * 4 + q) + khalf * 8) =
+            make_uint2(pack_bf16x2(acc[j][4 * q], acc[j][4 * q + 1]),
+                       pack_bf16x2(acc[j][4 * q + 2], acc[j][4 * q + 3]));
   }
-  store_pass<32 * MB, RBY>(epi, args.C + tc.n0 + wave * NB * 32, args.ldc, tc.p_begin, tc.p_end,
-                           lane);
+  __syncthreads();
+  const int tid = threadIdx.x;
+  if constexpr (MODE == 0 || MODE == 5) {  // 256-byte rows: 16 threads a row
+    uint16_t* const dst = MODE == 0 ? args.C : args.C2;
+    const int ld = MODE == 0 ? args.ldc : args.ldc2;
+#pragma unroll
+    for (int it = 0; it < 2 * MB; ++it) {
+      const int r = it * 16 + (tid >> 4), c = tid & 15;
+      const uint4 v = *reinterpret_cast<const uint4*>(at256(r, c));
+      if (tc.p_begin + r < tc.p_end)
+        store16_nt(dst + int64_t(tc.p_begin + r) * ld + tc.n0 + c * 8, v);
+    }
+  }
+  if constexpr (SWIGLU) {  // 128-byte rows: 8 threads a row
+#pragma unroll
+    for (int it = 0; it < MB; ++it) {
+      const int r = it * 32 + (tid >> 3), c = tid & 7;
+      const uint4 v = *reinterpret_cast<const uint4*>(at128(r, c));
+      if (tc.p_begin + r < tc.p_end)
+        store16_nt(args.C + int64_t(tc.p_begin + r) * args.ldc + tc.n0 / 2 + c * 8, v);
+    }
+  }
+  if constexpr (MODE == 4) {
+    // dGU = dh times the forward's factors (the persistent kernel's MODE 4), zeros
+    // in the rows from the expert's count on
+    const int p_valid = off(tc.e + 1);
+    const int64_t ld = args.ldc;
+    uint4 va[2 * MB], vb[2 * MB];
+    const int c = tid & 15;
+    const int f = tc.n0 + c * 8;
+    const int fcol = (f >> 5) * 64 + (f & 31);
+#pragma unroll
+    for (int it = 0; it < 2 * MB; ++it) {
+      const int p = tc.p_begin + it * 16 + (tid >> 4);
+      // padding rows read row 0 (valid whenever the launch has rows), unused
+      const uint16_t* src = args.aux + int64_t(p < p_valid ? p : 0) * ld + fcol;
+      va[it] = *reinterpret_cast<const uint4*>(src);
+      vb[it] = *reinterpret_cast<const uint4*>(src + 32);
+    }
+#pragma unroll
+    for (int it = 0; it < 2 * MB; ++it) {
+      const int r = it * 16 + (tid >> 4);
+      const uint4 v = *reinterpret_cast<const uint4*>(at256(r, c));
+      if (tc.p_begin + r < tc.p_end) {
+        const bool valid = tc.p_begin + r < p_valid;
+        const uint32_t dv[4] = {v.x, v.y, v.z, v.w};
+        const uint32_t av[4] = {va[it].x, va[it].y, va[it].z, va[it].w};
+        const uint32_t bv[4] = {vb[it].x, vb[it].y, vb[it].z, vb[it].w};
+        uint32_t og[4], ou[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float d0 = __uint_as_float(dv[w] << 16);
+          const float d1 = __uint_as_float(dv[w] & 0xffff0000u);
+          const uint32_t g = pack_bf16x2(d0 * __uint_as_float(av[w] << 16),
+                                         d1 * __uint_as_float(av[w] & 0xffff0000u));
+          const uint32_t u = pack_bf16x2(d0 * __uint_as_float(bv[w] << 16),
+                                         d1 * __uint_as_float(bv[w] & 0xffff0000u));
+          og[w] = valid ? g : 0u;
+          ou[w] = valid ? u : 0u;
+        }
+        uint16_t* dst = args.C + (int64_t(tc.a_row) + r) * ld + fcol;
+        store16_nt(dst, make_uint4(og[0], og[1], og[2], og[3]));
+        store16_nt(dst + 32, make_uint4(ou[0], ou[1], ou[2], ou[3]));
+      }
+    }
+  }
 }
 
-template <int MAXMB, int NB, int OCC, bool PADA>
+template <int MAXMB, int OCC, int MODE, bool DROP, bool PADA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void
 grouped_gemm_ring_kernel(GemmArgs args) {
-  constexpr int SMEM = 160 * 1024 / OCC;
+  constexpr int SMEM = 160 * 1024 / OCC / 1024 * 1024;
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];
-  constexpr int BN = 128 * NB;
   const Offsets off = load_offsets(args.offsets, args.n_experts);
-  const int ntn = args.Nout / BN;
+  const int ntn = args.Nout / 128;
   int total = 0;
-  for (int e = 0; e < args.n_experts; ++e)
-    total += (((expert_rows(args, off, e) + 31) / 32 + MAXMB - 1) / MAXMB) * ntn;
+  for (int e = 0; e < args.n_experts; ++e) {
+    int nb, mt, zt;
+    ring_blocks<MAXMB, MODE>(args, off, e, nb, mt, zt);
+    total += (mt + zt) * ntn;
+  }
+  // XCD x (workgroup b runs on XCD b % 8) takes a contiguous eighth of the tiles
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
   if (lo + slot >= hi) return;
   RingTile tc;
-  ring_decode<MAXMB, PADA>(args, off, lo + slot, ntn, BN, tc);
-  if (tc.mb == 1) ring_tile<1, NB, SMEM, PADA>(args, tc, smem);
-  if constexpr (MAXMB >= 2) if (tc.mb == 2) ring_tile<2, NB, SMEM, PADA>(args, tc, smem);
-  if constexpr (MAXMB >= 3) if (tc.mb == 3) ring_tile<3, NB, SMEM, PADA>(args, tc, smem);
-  if constexpr (MAXMB >= 4) if (tc.mb == 4) ring_tile<4, NB, SMEM, PADA>(args, tc, smem);
+  ring_decode<MAXMB, MODE, PADA>(args, off, lo + slot, ntn, tc);
+  if constexpr (MODE == 4) {
+    if (tc.mb == 0) {
+      ring_zero_tile(args, tc);
+      return;
+    }
+  }
+  if (tc.mb == 1) ring_tile<1, SMEM, MODE, DROP, PADA>(args, tc, off, smem);
+  if constexpr (MAXMB >= 2)
+    if (tc.mb == 2) ring_tile<2, SMEM, MODE, DROP, PADA>(args, tc, off, smem);
+  if constexpr (MAXMB >= 3)
+    if (tc.mb == 3) ring_tile<3, SMEM, MODE, DROP, PADA>(args, tc, off, smem);
+  if constexpr (MAXMB >= 4)
+    if (tc.mb == 4) ring_tile<4, SMEM, MODE, DROP, PADA>(args, tc, off, smem);
 }
 
 }  // namespace
@@ -1523,6 +1712,92 @@ void launch_persist(unsigned grid, const GemmArgs& a, hipStream_t st) {
         dim3(grid), dim3(256), 0, st, a);
 }
 
+// Small M: fewer rows than one and a half 256 x 256 tiles per CU would take if
+// packed (the per-expert counts stay on the device).
+inline bool small_m(int64_t rows, int nout, unsigned ncu) {
+  return rows * nout < int64_t(3 * ncu / 2) * 256 * 256;
+}
+
+template <int MAXMB, int OCC, int MODE, bool DROP, bool PADA>
+void launch_ring_tiles(const GemmArgs& a, int64_t rows, hipStream_t st) {
+  // tiles: sum_e ceil(ceil(cnt_e / 32) / MAXMB) <= rows / (32 MAXMB) + E per column,
+  // and (MODE 4) at most two zero tiles per expert (383 rows at most)
+  const int64_t mt = (rows + 32 * MAXMB - 1) / (32 * MAXMB) + (MODE == 4 ? 3 : 1) * a.n_experts;
+  const unsigned grid = unsigned((mt * (a.Nout / 128) + 7) / 8 * 8);
+  hipLaunchKernelGGL((grouped_gemm_ring_kernel<MAXMB, OCC, MODE, DROP, PADA>), dim3(grid),
+                     dim3(256), 0, st, a);
+}
+
+// 32-row blocks of an expert with the mean row count and two standard deviations
+// of uniform routing more (the counts themselves stay on the device).
+inline int64_t ring_mean_blocks(int64_t rows, int n_experts) {
+  const double mean = double(rows) / n_experts;
+  const int64_t m = int64_t(mean + (n_experts > 1 ? 2.0 * std::sqrt(mean) : 0.0));
+  return std::max<int64_t>(1, (m + 31) / 32);
+}
+
+// The ring kernel's tile height: the smallest whose tiles do not
+// outnumber the CUs, else the smallest with at most two per CU, else 128 rows.
+// Fewer rows per tile keep more CUs pulling the weight stream; a tile more than
+// the resident workgroups costs a whole tile's time (down, 4,096 rows: 432
+// 64-row tiles 33 us, 288 96-row ones 41).  128- and 96-row tiles with at most
+// one per CU take all of its LDS (OCC = 1: 26.6 against 33.5 us at 1,554 rows,
+// 96-row tiles; two stages of half the LDS leave one in flight), smaller ones
+// start sooner with half (one expert, 300 x 768 x 768: 6.2 against 6.9 us).
+template <bool PADA>
+void launch_ring(const GemmArgs& a, int64_t rows, unsigned ncu, hipStream_t st) {
+  const int64_t nb = ring_mean_blocks(rows, a.n_experts);
+  auto tiles = [&](int mb) { return (nb + mb - 1) / mb * a.n_experts * (a.Nout / 128); };
+  int mb = 1, per_cu = 1;
+  while (mb < 4 && tiles(mb) > int64_t(ncu)) ++mb;
+  if (tiles(mb) > int64_t(ncu)) {
+    per_cu = 2;
+    for (mb = 1; mb < 4 && tiles(mb) > 2 * int64_t(ncu);) ++mb;
+  }
+  if (mb == 1)
+    launch_ring_tiles<1, 2, 0, false, PADA>(a, rows, st);
+  else if (mb == 2)
+    launch_ring_tiles<2, 2, 0, false, PADA>(a, rows, st);
+  else if (mb == 3 && per_cu == 1)
+    launch_ring_tiles<3, 1, 0, false, PADA>(a, rows, st);
+  else if (mb == 3)
+    launch_ring_tiles<3, 2, 0, false, PADA>(a, rows, st);
+  else if (per_cu == 1)
+    launch_ring_tiles<4, 1, 0, false, PADA>(a, rows, st);
+  else
+    launch_ring_tiles<4, 2, 0, false, PADA>(a, rows, st);
+}
+
+// Whether a gate|up (MODE 1 / 5) or dh (MODE 4) launch takes the ring kernel: its
+// experts have at most max_blocks 32-row blocks (mean and two standard deviations
+// of uniform routing), or its 256 x 256 tiles would leave half the CUs idle.
+// Beyond that the persistent tiles win, whose 128 x 128 wave blocks read half the
+// LDS bytes per MFMA.  Measured, 16 experts, d = 768, F = 3,072, weights from
+// HBM (persistent -> ring): gate|up 48 tokens 45.9 -> 30.0 us, 400 43.7 -> 32.5,
+// 777 (4 blocks) 44.5 -> 43.2, 1,100 (5 blocks) 45.4 -> 49.8; with factors and
+// dropout 54.5 -> 34.7, 54.4 -> 38.2, 55.2 -> 49.7, 60.7 -> 60.6; dh 56.0 ->
+// 25.0, 52.0 -> 26.7, 51.7 -> 33.2, 50.9 -> 34.6, 2,048 tokens (9 blocks) 60.9 ->
+// 57.5, 3,000 69.3 -> 78.6.  8 experts, d = 256, F = 1,024, 1,100 tokens: gate|up
+// 14.0 -> 8.3, dh 18.5 -> 8.7.
+inline bool ring_wide(const GemmArgs& a, int64_t nk, int max_blocks, unsigned ncu, int* nb_out) {
+  const int64_t nb = ring_mean_blocks(nk, a.n_experts);
+  *nb_out = int(std::min<int64_t>(nb, 1 << 20));
+  const int64_t m256 = (nk + a.n_experts - 1) / a.n_experts;
+  return nb <= max_blocks ||
+         (m256 + 255) / 256 * a.n_experts * (a.Nout / 256) * 2 <= int64_t(ncu);
+}
+
+// The ring launch of such a product: tiles of 3 blocks where that deals an
+// expert's blocks more evenly than 4 (5, 6 and 9 blocks).
+template <int MODE, bool DROP, bool PADA>
+void launch_ring_wide(const GemmArgs& a, int64_t nk, int nb, hipStream_t st) {
+  const int mt = (nb + 3) / 4;
+  if ((nb + mt - 1) / mt == 3)
+    launch_ring_tiles<3, 2, MODE, DROP, PADA>(a, nk, st);
+  else
+    launch_ring_tiles<4, 2, MODE, DROP, PADA>(a, nk, st);
+}
+
 // Token rows per m-tile of the gate|up GEMMs: 192 when, at the launch's mean
 // rows per expert, 192-row tiles pad to at least 10 % fewer rows than 256-row
 // ones (a shard's share of the tokens: 569 rows per expert fill three tiles
@@ -1568,6 +1843,11 @@ hipError_t launch_gate_up(const uint16_t* xb, const int32_t* perm, const int32_t
   a.ldc = s.d_ff;
   a.ldc2 = 2 * s.d_ff;
   if (a.K < G5_GU_STAGES * G5_GU_BK) return hipErrorInvalidValue;
+  int nb = 0;
+  if (gu == nullptr && ring_wide(a, nk, 4, unsigned(device_cu_count()), &nb)) {
+    launch_ring_wide<1, false, false>(a, nk, nb, st);
+    return hipGetLastError();
+  }
   // 192-row tiles for the inference gate|up at small mean expert counts
   const bool bm192 = gu == nullptr && gate_up_bm(nk, s.n_experts, a.K) == 192;
   const unsigned grid = bm192 ? grid_bound<192, 256>(nk, s.n_experts, a.Nout)
@@ -1614,16 +1894,26 @@ hipError_t launch_gate_up_ab(const uint16_t* xb, const int32_t* perm, const int3
   a.ldc = s.d_ff;
   a.ldc2 = 2 * s.d_ff;
   if (a.K < G5_GU_STAGES * G5_GU_BK) return hipErrorInvalidValue;
+  if (drop.on) {
+    a.drop_seed_lo = drop.seed_lo;
+    a.drop_seed_hi = drop.seed_hi;
+    a.drop_thr = drop.thr;
+    a.drop_scale = drop.scale;
+  }
+  int nb = 0;
+  if (ring_wide(a, nk, 4, unsigned(device_cu_count()), &nb)) {
+    if (drop.on)
+      launch_ring_wide<5, true, false>(a, nk, nb, st);
+    else
+      launch_ring_wide<5, false, false>(a, nk, nb, st);
+    return hipGetLastError();
+  }
   const bool bm192 = gate_up_bm(nk, s.n_experts, a.K) == 192;
   const unsigned tiles = bm192 ? grid_bound<192, 256>(nk, s.n_experts, a.Nout)
                                : grid_bound<256, 256>(nk, s.n_experts, a.Nout);
   const unsigned grid = std::min(tiles, unsigned(device_cu_count()));
   a.xs = xcd_split(4 + (drop.on ? 2 : 0) + (bm192 ? 1 : 0), grid, a.K, a.Nout, st);
   if (drop.on) {
-    a.drop_seed_lo = drop.seed_lo;
-    a.drop_seed_hi = drop.seed_hi;
-    a.drop_thr = drop.thr;
-    a.drop_scale = drop.scale;
     if (bm192)
       launch_gate_up192<5, true>(grid, a, st);
     else
@@ -1660,62 +1950,17 @@ hipError_t launch_dh_swiglu(const uint16_t* dy_pad, int kmax, const int32_t* off
   a.K = d;
   a.Nout = F;
   a.ldc = 2 * F;
+  int nb = 0;
+  if (ring_wide(a, nk, 8, unsigned(device_cu_count()), &nb)) {
+    launch_ring_wide<4, false, true>(a, nk, nb, st);
+    return hipGetLastError();
+  }
   const unsigned grid = std::min(grid_bound<256, 256>(prows, E, F), unsigned(device_cu_count()));
   launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 4, true>(grid, a, st);
   return hipGetLastError();
 }
 
 namespace {
-
-// Small M: fewer rows than one and a half 256 x 256 tiles per CU would take if
-// packed (the per-expert counts stay on the device).
-inline bool small_m(int64_t rows, int nout, unsigned ncu) {
-  return rows * nout < int64_t(3 * ncu / 2) * 256 * 256;
-}
-
-template <int MAXMB, int OCC, bool PADA>
-void launch_ring_tiles(const GemmArgs& a, int64_t rows, hipStream_t st) {
-  // tiles: sum_e ceil(ceil(cnt_e / 32) / MAXMB) <= rows / (32 MAXMB) + E per column
-  const int64_t mt = (rows + 32 * MAXMB - 1) / (32 * MAXMB) + a.n_experts;
-  const unsigned grid = unsigned((mt * (a.Nout / 128) + 7) / 8 * 8);
-  hipLaunchKernelGGL((grouped_gemm_ring_kernel<MAXMB, 1, OCC, PADA>), dim3(grid), dim3(256), 0,
-                     st, a);
-}
-
-// The ring kernel's tile height: the smallest whose tiles (for experts of the
-// mean row count and two standard deviations of uniform routing more) do not
-// outnumber the CUs, else the smallest with at most two per CU, else 128 rows.
-// Fewer rows per tile keep more CUs pulling the weight stream; a tile more than
-// the resident workgroups costs a whole tile's time (down, 4,096 rows: 432
-// 64-row tiles 33 us, 288 96-row ones 41).  128- and 96-row tiles with at most
-// one per CU take all of its LDS (OCC = 1: 26.6 against 33.5 us at 1,554 rows,
-// 96-row tiles; two stages of half the LDS leave one in flight), smaller ones
-// start sooner with half (one expert, 300 x 768 x 768: 6.2 against 6.9 us).
-template <bool PADA>
-void launch_ring(const GemmArgs& a, int64_t rows, unsigned ncu, hipStream_t st) {
-  const double mean = double(rows) / a.n_experts;
-  const int64_t m = int64_t(mean + (a.n_experts > 1 ? 2.0 * std::sqrt(mean) : 0.0));
-  const int64_t nb = std::max<int64_t>(1, (m + 31) / 32);
-  auto tiles = [&](int mb) { return (nb + mb - 1) / mb * a.n_experts * (a.Nout / 128); };
-  int mb = 1, per_cu = 1;
-  while (mb < 4 && tiles(mb) > int64_t(ncu)) ++mb;
-  if (tiles(mb) > int64_t(ncu)) {
-    per_cu = 2;
-    for (mb = 1; mb < 4 && tiles(mb) > 2 * int64_t(ncu);) ++mb;
-  }
-  if (mb == 1)
-    launch_ring_tiles<1, 2, PADA>(a, rows, st);
-  else if (mb == 2)
-    launch_ring_tiles<2, 2, PADA>(a, rows, st);
-  else if (mb == 3 && per_cu == 1)
-    launch_ring_tiles<3, 1, PADA>(a, rows, st);
-  else if (mb == 3)
-    launch_ring_tiles<3, 2, PADA>(a, rows, st);
-  else if (per_cu == 1)
-    launch_ring_tiles<4, 1, PADA>(a, rows, st);
-  else
-    launch_ring_tiles<4, 2, PADA>(a, rows, st);
-}
 
 // The MODE 0 products (A rows in place, or per-expert padded with PADA).
 template <bool PADA>

@@ -58,3 +58,76 @@ def test_ring_equals_persistent_tiles(cuda_device, K, n_out, counts, packed):
         # one bf16 rounding (2^-9 relative, half an ulp) of an fp32 sum of K products of
         # about N(0, 1/K): K fp32 roundings of partial sums of about 1
         assert (err <= ref.abs() * 2.0 ** -8 + K * 2.0 ** -24 * 4).all()
+
+
+@pytest.mark.parametrize("n,d,F,E,k,p", [
+    (1, 768, 3072, 16, 2, 0.1),      # two rows in all
+    (130, 768, 3072, 16, 2, 0.0),    # one block per expert
+    (777, 768, 3072, 16, 2, 0.1),    # up to four blocks, the last partial
+    (1000, 256, 1024, 8, 2, 0.1),    # three-block tiles
+    (96, 128, 128, 4, 1, 0.0),       # the smallest d and F: two k-steps, two n-tiles
+])
+def test_ring_gate_up_equals_persistent_tiles(cuda_device, n, d, F, E, k, p):
+    """The gate|up products of a few tokens (ring kernel) equal the same tokens' rows in a
+    batch that takes the persistent tiles, bit for bit: h, and where the training forward
+    keeps them (d and F multiples of 256) the SwiGLU factors, under one dropout mask (it is
+    keyed on the token and slot)."""
+    print(f"ring gate|up n={n} d={d} F={F} E={E} k={k} p={p}", flush=True)
+    g = torch.Generator(device=cuda_device).manual_seed(n + d)
+    big = 24000 if d < 768 else 6000
+    r = lambda *s, std=1.0: (torch.randn(*s, device=cuda_device, generator=g) * std).bfloat16()
+    x, wr = r(big, d), r(E, d, std=0.05)
+    wgu, wd = r(E, 2 * F, d, std=0.02), r(E, d, F, std=0.02)
+    train = d % 256 == 0 and F % 256 == 0
+    rows = []
+    for m in (n, big):
+        if train:
+            out = ops.moe_forward_train(x[:m], wr, wgu, wd, k, dropout=(p, 77) if p else None,
+                                        return_h=True, factors=True)
+            inv, ops_rows = out[6][:n * k].long(), (out[9], out[8])
+            rows.append([t[inv] for t in ops_rows])
+        idx, _, _, off, perm, inv = ops.route(x[:m], wr, k)
+        _, h = ops.expert_swiglu(x[:m], perm, off, wgu, wd, k, return_h=True)
+        rows.append([h[inv[:n * k].long()]])
+    torch.cuda.synchronize()
+    half = len(rows) // 2
+    for small, large in zip(rows[:half], rows[half:]):
+        for a, b in zip(small, large):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("counts", [[0, 1, 31, 32, 33, 64, 0, 129], [383, 0, 97, 2],
+                                    [0, 0, 0, 5]])
+@pytest.mark.parametrize("kmax", [0, 384])
+def test_ring_dh_swiglu_equals_staged(cuda_device, counts, kmax):
+    """The dh product with the SwiGLU backward of a few rows (ring kernel): the staged dh
+    times the factors in fp32, bit for bit, zeros in every padding row that the weight
+    gradient reads and nothing written after them."""
+    import ctypes
+
+    from genet5_amd import _lib
+    d, F, E = 256, 512, len(counts)
+    print(f"ring dh counts={counts} kmax={kmax}", flush=True)
+    g = torch.Generator(device=cuda_device).manual_seed(sum(counts) + kmax)
+    rows = sum(counts)
+    off, t_off = _offsets(counts, cuda_device)
+    wrows = [max(384, -(-c // 192) * 192) for c in counts]
+    starts = [e * kmax if kmax else sum(wrows[:e]) for e in range(E)]
+    prows = E * kmax if kmax else ops.packed_rows(rows, E)
+    dy = torch.randn(prows + ops.ROW_PAD, d, device=cuda_device, generator=g).bfloat16()
+    wdt = (torch.randn(E, F, d, device=cuda_device, generator=g) * 0.05).bfloat16()
+    fac = torch.randn(rows, 2 * F, device=cuda_device, generator=g).bfloat16()
+    got = torch.full((prows + ops.ROW_PAD, 2 * F), 7.0, device=cuda_device).bfloat16()
+    shape = _lib.make_shape(rows, d, F, E, 1, _lib.DTYPE_BF16)
+    _lib.call("g5moe_dh_swiglu_backward", ops._ptr(dy), kmax, ops._ptr(t_off), ops._ptr(wdt),
+              ops._ptr(fac), ops._ptr(got), ctypes.byref(shape), ops._stream(cuda_device))
+    dh = ops.grouped_gemm_padded(dy, kmax, rows, t_off, wdt).float()
+    want = torch.full_like(got, 7.0)
+    fv = fac.view(rows, F // 32, 2, 32).float()
+    prod = (dh.view(rows, F // 32, 1, 32) * fv).reshape(rows, 2 * F).bfloat16()
+    for e in range(E):
+        want[starts[e]:starts[e] + wrows[e]] = 0
+        want[starts[e]:starts[e] + counts[e]] = prod[off[e]:off[e + 1]]
+    torch.cuda.synchronize()
+    # values: a zero product may carry either sign
+    assert torch.equal(got.float(), want.float())
