@@ -11,8 +11,21 @@
 //
 // Work split: one workgroup of 4 waves per (128-query block, head, sequence);
 // wave w owns queries q0 + 32w .. q0 + 32w + 31.  Keys stream through LDS in
-// blocks of 64 (K row-major, V transposed), double-buffered, one barrier per
-// block.
+// blocks of 64, a ring of three (K, V) tiles filled by LDS DMA (no staging
+// registers, no LDS writes), one barrier per block: after the softmax, when the
+// next tile has landed and every wave holds its V operands of this one; the next
+// block's K operands are read behind the output product.  Each wave walks its
+// blocks as runs of one kind (before its queries, across them, after them, the
+// partial last one), so that the block loops carry no branches.
+//
+// What bounds it: with two waves per SIMD the matrix core and the VALU are each
+// busy about half of the cycles and the clock falls to 1.9 GHz under the power
+// limit; per 64-key block and wave 22 MFMAs (704 cycles) against 32 exps (8
+// cycles each), 32 multiplies, 16 conversions and about 30 more.  At 8 x 4,550
+// tokens, 12 heads (captured loops, one GPU, against the register-staged,
+// branching loop with a multiplied-out bias before it): ALiBi 449 -> 377 us, with
+// twice the scores (online loop) 534 -> 453, no ALiBi 745 -> 591 (861 TFLOP/s) and
+// 789 -> 652; 2 x 2,275 without ALiBi 66 -> 49.
 //
 // MFMA layout (v_mfma_f32_32x32x16_bf16): scores are formed transposed,
 // S^T = K . Q^T, with the key block as the A operand and the wave's queries as
@@ -24,12 +37,10 @@
 // movement (a lane's eight probabilities of a 16-key chunk are its own
 // accumulator elements), provided V^T's key order inside each 16-key chunk is
 // the one those elements carry: key r at position r with bits 2 and 3
-// swapped.  The LDS copy of V is written transposed in that order.
+// swapped.  V's transposing LDS reads fetch the keys in that order.
 //
-// LDS rows are padded to 144 bytes (K rows and V^T rows of 64 bf16): the 16
-// rows a 16-lane group of a fragment read touches then start 36 banks apart
-// (mod 64), which covers all 64 banks with 16-byte reads, and every tile write
-// is a base address plus an immediate offset.
+// LDS rows are 128 bytes, their 16-byte chunks swizzled by the row (see the tile
+// loads) so that the fragment reads hit distinct banks.
 //
 // Block skipping under ALiBi: with key norms bounded by KM (the largest of the
 // per-64-token-block maxima a pre-pass writes, over the blocks that cover the
@@ -48,22 +59,24 @@
 //   and every |s * sc| of the workgroup within 32): p = 2^(t - mref) with the
 //   lane's fixed upper bound mref = sc * |q| * KM >= t.  The row's largest term
 //   is at least its diagonal's, >= -mref, so no probability that matters
-//   underflows and no running maximum or rescaling is needed.  On a key block
-//   wholly on one side of the wave's queries (and inside the sequence) the
-//   ALiBi bias and -mref enter the score product as one more MFMA k-chunk
-//   (key offsets against bf16 splits of the slope and of the lane's
-//   constant), so a probability costs one multiply and one exp; the row sums
-//   that normalise the output come from an all-ones MFMA operand against P^T
+//   underflows and no running maximum or rescaling is needed; the row sums that
+//   normalise the output come from an all-ones MFMA operand against P^T
 //   (the sums of the bf16 probabilities the output product weights; the fp32
 //   sums are kept only when softmax_lse is asked for).
-// * Online (otherwise): running maximum, rescaled output and row sum.  On a
-//   one-sided block bias = c_blk +/- c_r with c_r = -slope * log2(e) * (key
-//   offset inside the block) held in registers and c_blk a per-lane scalar,
-//   so the bias costs nothing beyond the score's own fused multiply-add.
+// * Online (otherwise): running maximum, rescaled output and row sum.
+//
+// On a key block wholly on one side of the wave's queries (and inside the
+// sequence) the ALiBi bias (and the reference loop's -mref) enters the score
+// product as one more MFMA k-chunk (key offsets against bf16 splits of the slope
+// and of the lane's constant), so a probability costs one multiply (or fused
+// multiply-add) and one exp.
 //
 // Blocks that straddle the diagonal or the sequence end take the exact
 // per-element |i - j| path with masking in both loops.
-#include "g5moe_internal.h"
+#include <algorithm>
+#include <type_traits>
+
+#include "gemm_common.h"
 
 namespace g5moe {
 namespace {
@@ -75,13 +88,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kHeadDim = 64;
 constexpr int kBQ = 128;   // queries per workgroup (32 per wave)
 constexpr int kBKV = 64;   // keys per LDS block
-constexpr int kRowBytes = kHeadDim * 2 + 16;      // 144: padded K row
-constexpr int kTileBytes = kBKV * kRowBytes;      // 9 KB
-// V rows (one key each) 192 bytes apart: the four keys a transposing read's
-// 16-lane group covers start at a multiple of 4, so their 64-byte row pieces
-// land in four distinct quarters of the 64 banks.
-constexpr int kVRowBytes = kHeadDim * 2 + 64;
-constexpr int kVTileBytes = kBKV * kVRowBytes;    // 12 KB
+constexpr int kRowBytes = kHeadDim * 2;           // one key's K or V row in LDS
+constexpr int kTileBytes = kBKV * kRowBytes;      // 8 KB
+constexpr int kStageBytes = 2 * kTileBytes;       // K tile, then V tile
+constexpr int kStages = 3;
 constexpr float kSkipMargin = 64.0f;              // skipped keys have p < 2^-64
 constexpr float kFixedGap = 64.0f;                // reference-max loop: row maximum >= 2^-64
 constexpr float kLog2e = 1.4426950408889634f;
@@ -105,9 +115,6 @@ struct AttnArgs {
   int64_t total;
 };
 
-// Byte offset of 16-byte chunk c of LDS row r.
-__device__ __forceinline__ int lds_off(int row, int chunk) { return row * kRowBytes + chunk * 16; }
-
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4* lds_i16x4_p;
 
@@ -119,12 +126,23 @@ __device__ __forceinline__ i16x4 read_tr(const char* p) {
       uintptr_t((__attribute__((address_space(3))) const char*)p)));
 }
 
-// LSE: softmax_lse is written (a.lse != nullptr).
-template <bool LSE>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2)))
+// LDS DMA with a 64-bit address per lane (gemm::lds_dma16_s with a scalar base
+// otherwise).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_dma16_v(const char* addr, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :: "v"(addr), "s"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// LSE: softmax_lse is written (a.lse != nullptr).  WIDE: a token stride of k or v
+// too large for 32-bit offsets inside a 64-key tile.
+template <bool LSE, bool WIDE>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
 void attn_fwd_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) char ksm[2][kTileBytes];   // K rows
-  __shared__ __attribute__((aligned(16))) char vsm[2][kVTileBytes];  // V rows
+  __shared__ __attribute__((aligned(1024))) char ring[kStages * kStageBytes];
 
   const int z = blockIdx.z;
   const int hq = blockIdx.y;
@@ -157,6 +175,14 @@ void attn_fwd_kernel(AttnArgs a) {
     for (int kc = 0; kc < 4; ++kc) {
       const u32x4 raw = ok ? *reinterpret_cast<const u32x4*>(qp + 16 * kc) : u32x4{0, 0, 0, 0};
       qf[kc] = __builtin_bit_cast(bf16x8, raw);
+    }
+    // the queries landed: a load the compiler still counted as in flight at the
+    // block loop would make every block wait for its tile loads (vmcnt 0)
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) {
+      u32x4 w = __builtin_bit_cast(u32x4, qf[kc]);
+      asm volatile("" : "+v"(w));
+      qf[kc] = __builtin_bit_cast(bf16x8, w);
     }
   }
   // Key blocks this workgroup visits: [n_lo, n_hi] (all of them without ALiBi
@@ -214,69 +240,81 @@ void attn_fwd_kernel(AttnArgs a) {
     mref = sc * __builtin_sqrtf(ss_own) * kmx;
   }
 
-  // Tile loaders: thread t moves rows (t >> 3) and (t >> 3) + 32, chunk t & 7
-  // (eight threads per 128-byte row), of K and of V.  Rows past the sequence
-  // end are zero (masked keys then meet finite values only).
-  const int k_row = tid >> 3, k_chunk = tid & 7;
-  const uint16_t* kbase = a.k + int64_t(s0) * a.k_tok + hk * a.k_head;
-  const uint16_t* vbase = a.v + int64_t(s0) * a.v_tok + hk * a.v_head;
-  // per-lane element offsets inside a tile (the tile's base is block-uniform)
-  const int64_t k_off0 = int64_t(k_row) * a.k_tok + k_chunk * 8;
-  const int64_t k_off1 = k_off0 + 32 * a.k_tok;
-  const int64_t v_off0 = int64_t(k_row) * a.v_tok + k_chunk * 8;
-  const int64_t v_off1 = v_off0 + 32 * a.v_tok;
-  u32x4 kreg[2], vreg[2];
-  auto load_k = [&](int j0) __attribute__((always_inline)) {
-    const uint16_t* kt = kbase + int64_t(j0) * a.k_tok;
+  // Tile loads, straight to LDS: DMA instruction i (0, 1: K, 2, 3: V) of a wave
+  // fills the 8 key rows of block 4 (i % 2) + wave of a tile.  K's chunk c of row r
+  // goes to c ^ ((r >> 1) & 7) (16-lane groups of a fragment read then hit 16
+  // distinct bank groups), V's to c ^ 2 (r & 3) (the four keys of a transposing
+  // read in four distinct ones).  Rows past the sequence end repeat its last row:
+  // their scores are masked, and V's are cleared before they are read.
+  const int lrow = lane >> 3;
+  const uint32_t k_ch = uint32_t((lane & 7) ^ (((wave & 1) * 4 + (lrow >> 1)) & 7)) * 16;
+  const uint32_t v_ch = uint32_t((lane & 7) ^ (2 * (lrow & 3))) * 16;
+  const char* const kbase =
+      reinterpret_cast<const char*>(a.k + int64_t(s0) * a.k_tok + hk * a.k_head);
+  const char* const vbase =
+      reinterpret_cast<const char*>(a.v + int64_t(s0) * a.v_tok + hk * a.v_head);
+  const int64_t k_tok2 = a.k_tok * 2, v_tok2 = a.v_tok * 2;
+  const uint32_t ring_lds = gemm::lds_addr(ring) + uint32_t(wave) * 1024;
+  // Lane offsets of the wave's rows in a whole tile and in the sequence's last one.
+  const int last_rows = L - (nblk - 1) * kBKV;
+  uint32_t koff[2][2], voff[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = (4 * i + wave) * 8 + lrow;
+    koff[0][i] = uint32_t(row) * uint32_t(k_tok2) + k_ch;
+    voff[0][i] = uint32_t(row) * uint32_t(v_tok2) + v_ch;
+    const int rl = min(row, last_rows - 1);
+    koff[1][i] = uint32_t(rl) * uint32_t(k_tok2) + k_ch;
+    voff[1][i] = uint32_t(rl) * uint32_t(v_tok2) + v_ch;
+  }
+  // The next tile to load (n_is, at kt / vt); past n_hi the last tile goes out
+  // again, into a buffer that no later block reads, so that every block issues
+  // four instructions and the waits are constants.
+  int n_is = n_lo;
+  const char* kt = kbase + n_lo * kBKV * k_tok2;
+  const char* vt = vbase + n_lo * kBKV * v_tok2;
+  auto issue = [&](uint32_t boff) __attribute__((always_inline)) {
+    const uint32_t dst = ring_lds + boff;
+    const bool last = n_is == nblk - 1;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const int kr = j0 + k_row + 32 * i;
-      kreg[i] = kr < L ? *reinterpret_cast<const u32x4*>(kt + (i == 0 ? k_off0 : k_off1))
-                       : u32x4{0, 0, 0, 0};
-    }
-  };
-  auto load_v = [&](int j0) __attribute__((always_inline)) {
-    const uint16_t* vt = vbase + int64_t(j0) * a.v_tok;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int vr = j0 + k_row + 32 * i;
-      vreg[i] = vr < L ? *reinterpret_cast<const u32x4*>(vt + (i == 0 ? v_off0 : v_off1))
-                       : u32x4{0, 0, 0, 0};
-    }
-  };
-  auto store_k = [&](int buf) __attribute__((always_inline)) {
-    char* Ks = ksm[buf];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      *reinterpret_cast<u32x4*>(Ks + lds_off(k_row + 32 * i, k_chunk)) = kreg[i];
-  };
-  auto store_v = [&](int buf) __attribute__((always_inline)) {
-    char* Vs = vsm[buf];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      *reinterpret_cast<u32x4*>(Vs + (k_row + 32 * i) * kVRowBytes + k_chunk * 16) = vreg[i];
-  };
-  auto load_tile = [&](int j0) __attribute__((always_inline)) {
-    load_k(j0);
-    load_v(j0);
-  };
-  auto store_tile = [&](int buf) __attribute__((always_inline)) {
-    store_k(buf);
-    store_v(buf);
-  };
-  // S^T = K . Q^T for the two 32-key halves of the block
-  auto scores = [&](const char* Ks, f32x16* s) __attribute__((always_inline)) {
-    const f32x16 zero16 = {};
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int kc = 0; kc < 4; ++kc) {
-        const bf16x8 kf =
-            *reinterpret_cast<const bf16x8*>(Ks + lds_off(32 * b + col, 2 * kc + half));
-        s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kc], kc == 0 ? zero16 : s[b], 0,
-                                                       0, 0);
+      if constexpr (WIDE) {
+        const int r0 = (4 * i + wave) * 8 + lrow;
+        const int row = last ? min(r0, last_rows - 1) : r0;
+        lds_dma16_v(kt + row * k_tok2 + k_ch, dst + i * 4096);
+        lds_dma16_v(vt + row * v_tok2 + v_ch, dst + kTileBytes + i * 4096);
+      } else {
+        gemm::lds_dma16_s(kt, last ? koff[1][i] : koff[0][i], dst + i * 4096);
+        gemm::lds_dma16_s(vt, last ? voff[1][i] : voff[0][i], dst + kTileBytes + i * 4096);
       }
     }
+    const bool more = n_is < n_hi;
+    n_is += more ? 1 : 0;
+    kt += more ? kBKV * k_tok2 : 0;
+    vt += more ? kBKV * v_tok2 : 0;
+  };
+  // K fragments of a block: keys 32 b + col, head dims 16 kc + 8 half .. + 8
+  const int k_row = col * kRowBytes;
+  const int k_sw = (col >> 1) & 7;
+  bf16x8 kf[2][4];
+  auto load_kf = [&](uint32_t boff) __attribute__((always_inline)) {
+    const char* Ks = ring + boff + k_row;
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        kf[b][kc] = *reinterpret_cast<const bf16x8*>(Ks + 32 * b * kRowBytes +
+                                                     ((2 * kc + half) ^ k_sw) * 16);
+  };
+  // S^T = K . Q^T for the two 32-key halves of the block
+  auto scores = [&](f32x16* s) __attribute__((always_inline)) {
+    const f32x16 zero16 = {};
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b][kc], qf[kc], kc == 0 ? zero16 : s[b],
+                                                       0, 0, 0);
   };
   // P^T operand of 16-key chunk c (chunk c = key block c / 2, elements
   // 8 (c % 2) .. +8): the lane's own probabilities, no data movement
@@ -285,234 +323,254 @@ void attn_fwd_kernel(AttnArgs a) {
                         pk[c >> 1][4 * (c & 1) + 2], pk[c >> 1][4 * (c & 1) + 3]};
     return __builtin_bit_cast(bf16x8, praw);
   };
-  // O^T += V^T . P^T over the four 16-key chunks.  The V^T operand of lane
-  // (col, half) for chunk c is head dim 32 mb + col at the keys its P^T elements
-  // hold, 16 c + 4 half + {0..3, 8..11}: two transposing reads of four keys
-  // each, lane k of a 16-lane group addressing key (k / 4) of the four and the
-  // four dims from 4 (k % 4) of the group's 16.
-  const int v_lane = (4 * half + ((lane & 15) >> 2)) * kVRowBytes +
-                     (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
-  auto out_product = [&](const char* Vs, const uint32_t (*pk)[8], f32x16* o)
-      __attribute__((always_inline)) {
+  // The V^T operand of lane (col, half) for chunk c is head dim 32 mb + col at the
+  // keys its P^T elements hold, 16 c + 4 half + {0..3, 8..11}: two transposing
+  // reads of four keys each, lane k of a 16-lane group addressing key (k / 4) of
+  // the four and the four dims from 4 (k % 4) of the group's 16, i.e. byte
+  // 8 (k % 2) of chunk 4 mb + 2 (group % 2) + (k % 4) / 2.  The chunk's swizzle
+  // 2 (key % 4) = 2 (k / 4) is the lane's own.
+  const int vk = (lane & 15) >> 2;
+  const int v_row = kTileBytes + (4 * half + vk) * kRowBytes + 8 * (lane & 1);
+  const int v_c = (2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (2 * vk);
+  const int v_lane[2] = {v_row + v_c * 16, v_row + (v_c ^ 4) * 16};
+  bf16x8 vf[4][2];
+  auto load_vf = [&](uint32_t boff) __attribute__((always_inline)) {
+    const char* Vs = ring + boff;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const bf16x8 pf = p_chunk(pk, c);
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int mb = 0; mb < 2; ++mb) {
-        const char* vp = Vs + v_lane + 16 * c * kVRowBytes + 64 * mb;
+        const char* vp = Vs + v_lane[mb] + 16 * c * kRowBytes;
         const i16x4 lo = read_tr(vp);
-        const i16x4 hi = read_tr(vp + 8 * kVRowBytes);
+        const i16x4 hi = read_tr(vp + 8 * kRowBytes);
         const i16x4 vv[2] = {lo, hi};
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, vv);
-        o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[mb], 0, 0, 0);
+        vf[c][mb] = __builtin_bit_cast(bf16x8, vv);
       }
-    }
   };
   // Exact per-element bias and sequence-end mask of a block that straddles the
   // wave's queries or the sequence end: t = s * sc - sl * |i - j|, -inf past L.
-  auto exact_terms = [&](const f32x16* s, int j0, float (*t)[16]) __attribute__((always_inline)) {
-    const float di = float(iq - j0);
+  auto exact_terms = [&](f32x16* s, int j0) __attribute__((always_inline)) {
+    // distances and limits from the lane's first key, so that each element's own
+    // offset is a literal
+    const float di = float(iq - j0 - 4 * half);
+    const int lim = L - j0 - 4 * half;
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int kr = 32 * b + 8 * (r >> 2) + 4 * half + (r & 3);
+        const int kr = 32 * b + 8 * (r >> 2) + (r & 3);
         const float bias = -sl * __builtin_fabsf(di - float(kr));
-        t[b][r] = j0 + kr < L ? __builtin_fmaf(s[b][r], sc, bias) : -__builtin_inff();
+        s[b][r] = kr < lim ? __builtin_fmaf(s[b][r], sc, bias) : -__builtin_inff();
       }
   };
 
-  f32x16 o[2];
+  f32x16 o[2] = {f32x16{}, f32x16{}};
+  // reference maximum, normalising sum, fp32 sum for lse
+  float m = fixed ? mref : -__builtin_inff(), l_tot = 0.0f, l_lse = 0.0f;
+
+  // The ALiBi bias of a block wholly on one side of the wave's queries as one more
+  // 16-deep MFMA chunk, in units of raw scores: with u = sl / sc, J the block's
+  // first key from the wave's first query (a multiple of 32) and kr a key's offset
+  // in the block, the bias over sc is -+u (J + kr) +- u col (keys after / before
+  // the query), so key rows
+  //   [kr, kr, kr, Jl, Jl, Jl, Jh, Jh | Jh, 1, 1, 1, 0, 0, 0, 0]
+  // (J = Jl + Jh, Jh a multiple of 8,192: all exact in bf16 up to 2^21 keys) meet
+  // query columns [u1, u2, u3, u1, u2, u3, u1, u2 | u3, c1, c2, c3, 0, ...] of one
+  // sign, u1 + u2 + u3 and c1 + c2 + c3 bf16 splits (exact to fp32 precision; bf16
+  // products are exact in the fp32 accumulation).  The reference-max loop puts
+  // -mref / sc into c.  Per block only the J words of the key rows change.
+  const bool chunk_ok = __builtin_amdgcn_readfirstlane(
+                            int(sc > 0.0f && sl >= 0.0f && sl < sc * 0x1p60f)) != 0;
+  auto bf16r = [](float x) __attribute__((always_inline)) -> float { return float(__bf16(x)); };
+  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) -> uint32_t {
+    return pack_bf16x2(lo, hi);
+  };
+  u32x4 qx[2];            // query columns: keys after, keys before
+  uint32_t kx01[2][2];    // key words 0 and 1 of the two 32-key halves
   {
-    const f32x16 zero16 = {};
-    o[0] = zero16;
-    o[1] = zero16;
-  }
-  float m, l_tot, l_lse;  // reference maximum, normalising sum, fp32 sum for lse
-
-  load_tile(n_lo * kBKV);
-  store_tile(n_lo & 1);
-  __syncthreads();
-
-  if (fixed) {
-    // Reference-max loop: p = 2^(t - mref) with the lane's fixed bound mref
-    // (t <= mref because the bias is <= 0; the row's largest term is at least
-    // its diagonal's, >= -mref, so p_max >= 2^-kFixedGap): no running maximum,
-    // no rescaling.  On a block wholly on one side of the wave's queries the
-    // bias and -mref ride in the score product as one more 16-deep MFMA
-    // chunk: key rows K' = [kr, kr, kr, 1, 1, 1, 0, 0] (kr the key's offset
-    // inside the block, exact in bf16) against query columns Q' = [-+u1, -+u2,
-    // -+u3, c1, c2, c3, 0, 0], where u1 + u2 + u3 = u = sl / sc (the slope in
-    // units of raw scores) and c1 + c2 + c3 = c = -u * |j0 - i| - mref / sc
-    // are bf16 splits (exact to fp32 precision; bf16 products are exact in
-    // the fp32 accumulation), so the accumulator holds s + (bias - mref) / sc
-    // and p = 2^(acc * sc).  The row sums come from the matrix cores too: an
-    // all-ones A operand against P^T adds sum_k bf16(p) to every element of
-    // lacc (the same bf16 probabilities the output product weights).
-    auto bf16r = [](float x) __attribute__((always_inline)) -> float { return float(__bf16(x)); };
-    const float u = sl / sc;
+    const float u = chunk_ok ? sl / sc : 0.0f;
     const float u1 = bf16r(u), u2 = bf16r(u - u1), u3 = bf16r(u - u1 - u2);
-    const float mref_s = mref / sc;
-    const __bf16 bz = __bf16(0.0f), b1 = __bf16(1.0f);
-    bf16x8 kx[2];
+    const float ref = fixed ? mref / sc : 0.0f;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const float sg = side == 0 ? -1.0f : 1.0f;
+      const float c = -sg * u * float(col) - ref;
+      const float c1 = bf16r(c), c2 = bf16r(c - c1), c3 = bf16r(c - c1 - c2);
+      const float a1 = sg * u1, a2 = sg * u2, a3 = sg * u3;
+      const u32x4 h0 = {pack2(a1, a2), pack2(a3, a1), pack2(a2, a3), pack2(a1, a2)};
+      const u32x4 h1 = {pack2(a3, c1), pack2(c2, c3), 0u, 0u};
+      qx[side] = half == 0 ? h0 : h1;
+    }
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const __bf16 kr = __bf16(float(32 * b + col));
-      const bf16x8 v = {kr, kr, kr, b1, b1, b1, bz, bz};
-      const bf16x8 zv = {bz, bz, bz, bz, bz, bz, bz, bz};
-      kx[b] = half == 0 ? v : zv;
+      const float kr = float(32 * b + col);
+      kx01[b][0] = half == 0 ? pack2(kr, kr) : pack2(0.0f, 1.0f);
+      kx01[b][1] = half == 0 ? pack2(kr, 0.0f) : pack2(1.0f, 1.0f);
     }
-    const bf16x8 ones = {b1, b1, b1, b1, b1, b1, b1, b1};
-    f32x16 lacc = {};
-    // softmax_lse wants the fp32 sum of the probabilities (lacc sums their bf16
-    // roundings, which the output product weights)
-    constexpr bool want_lse = LSE;
-    float psum = 0.0f;
-
-    for (int n = n_lo; n <= n_hi; ++n) {
-      const int buf = n & 1;
-      const int j0 = n * kBKV;
-      if (n < n_hi) load_tile(j0 + kBKV);
-      const char* Ks = ksm[buf];
-      const char* Vs = vsm[buf];
-      f32x16 s[2];
-      scores(Ks, s);
-
-      const bool inside = j0 + kBKV <= L;
-      const bool after = inside && j0 > wq_hi;              // every key > every query
-      const bool before = inside && j0 + kBKV - 1 < wq_lo;  // every key < every query
-      uint32_t pk[2][8];
-      // without ALiBi (u = 0) every block inside the sequence takes the chunk
-      if (after || before || (inside && sl == 0.0f)) {
-        const float c = -u * float(after ? j0 - iq : iq - j0) - mref_s;
-        const float c1 = bf16r(c), c2 = bf16r(c - c1), c3 = bf16r(c - c1 - c2);
-        const float su = after ? -1.0f : 1.0f;
-        const bf16x8 qv = {__bf16(su * u1), __bf16(su * u2), __bf16(su * u3), __bf16(c1),
-                           __bf16(c2),      __bf16(c3),      bz,              bz};
-        const bf16x8 zv = {bz, bz, bz, bz, bz, bz, bz, bz};
-        const bf16x8 qx = half == 0 ? qv : zv;
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kx[b], qx, s[b], 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(s[b][r] * sc);
-            const float p1 = __builtin_amdgcn_exp2f(s[b][r + 1] * sc);
-            if constexpr (want_lse) {
-              psum += p0;
-              psum += p1;
-            }
-            pk[b][r >> 1] = pack_bf16x2(p0, p1);
-          }
-      } else {
-        float t[2][16];
-        exact_terms(s, j0, t);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            const float p0 = __builtin_amdgcn_exp2f(t[b][r] - mref);
-            const float p1 = __builtin_amdgcn_exp2f(t[b][r + 1] - mref);
-            if constexpr (want_lse) {
-              psum += p0;
-              psum += p1;
-            }
-            pk[b][r >> 1] = pack_bf16x2(p0, p1);
-          }
-      }
-      out_product(Vs, pk, o);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, p_chunk(pk, c), lacc, 0, 0, 0);
-
-      if (n < n_hi) store_tile(buf ^ 1);
-      __syncthreads();
+  }
+  const uint32_t half0 = half == 0 ? 0xffffffffu : 0u;
+  const bool far = L > 8192;
+  // Adds the chunk; Jf: float(J) (its words' low bits are zero)
+  auto add_chunk = [&](f32x16* s, float Jf, const u32x4& q) __attribute__((always_inline)) {
+    uint32_t w0 = 0u, w3 = 0u;
+    float jl = Jf;
+    if (far) {
+      const float jh = __builtin_truncf(Jf * 0x1p-13f) * 0x1p13f;  // towards zero
+      jl = Jf - jh;
+      const uint32_t jb = __float_as_uint(jh);
+      w0 = (jb >> 16) & ~half0;
+      w3 = (jb | (jb >> 16)) & half0;
     }
-    m = mref;
-    l_tot = lacc[0];
-    l_lse = psum + __shfl_xor(psum, 32, 64);
-  } else {
-    // Online softmax: running maximum m, rescaled output and sum.
-    // c_r = -slope * log2(e) * (offset of element r's key inside the block)
-    float ck[2][16];
+    const uint32_t lb = __float_as_uint(jl);
+    const uint32_t w1 = lb & half0;
+    const uint32_t w2 = w1 | (w1 >> 16);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const u32x4 kx = {kx01[b][0] | w0, kx01[b][1] | w1, w2, w3};
+      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kx),
+                                                     __builtin_bit_cast(bf16x8, q), s[b], 0, 0, 0);
+    }
+  };
+  auto block_max = [](const f32x16* s) __attribute__((always_inline)) -> float {
+    float mx = s[0][0];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        ck[b][r] = -sl * float(32 * b + 8 * (r >> 2) + 4 * half + (r & 3));
-    m = -__builtin_inff();
-    float l = 0.0f;
+      for (int r = 0; r < 16; r += 2)
+        mx = __builtin_fmaxf(__builtin_fmaxf(mx, s[b][r]), s[b][r + 1]);
+    return mx;
+  };
 
-    for (int n = n_lo; n <= n_hi; ++n) {
-      const int buf = n & 1;
-      const int j0 = n * kBKV;
-      if (n < n_hi) load_tile(j0 + kBKV);
-      const char* Ks = ksm[buf];
-      const char* Vs = vsm[buf];
-      f32x16 s[2];
-      scores(Ks, s);
+  // The wave's blocks [n_lo, n_hi] in order: [n_lo, e0) and [e1, e2) by the fast
+  // path (whole blocks on one side of the wave's queries, or any whole block
+  // without ALiBi), [e0, e1) and a partial last block by the exact one.  Every
+  // wave of the workgroup runs every block, so the barriers pair up.
+  const int end = min(n_hi + 1, L / kBKV);
+  int e0, e1;
+  if (!chunk_ok) {
+    e0 = n_lo;
+    e1 = end;
+  } else if (sl == 0.0f) {
+    e0 = e1 = end;
+  } else {
+    e0 = min(wq_lo / kBKV, end);
+    e1 = min(wq_lo / kBKV + 1, end);
+  }
+  const bool tail = n_hi == nblk - 1 && last_rows < kBKV;
 
-      // t = s * sc + bias (base 2), block maximum, rescale, probabilities
-      const bool inside = j0 + kBKV <= L;
-      const bool after = inside && j0 > wq_hi;              // every key > every query
-      const bool before = inside && j0 + kBKV - 1 < wq_lo;  // every key < every query
-      float cblk;
-      float t[2][16];
-      if (after) {
-        cblk = -sl * float(j0 - iq);
+  uint32_t boff = 0;
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) t[b][r] = __builtin_fmaf(s[b][r], sc, ck[b][r]);
-      } else if (before) {
-        cblk = -sl * float(iq - j0);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) t[b][r] = __builtin_fmaf(s[b][r], sc, -ck[b][r]);
-      } else {
-        cblk = 0.0f;
-        exact_terms(s, j0, t);
-      }
-      float mx = t[0][0];
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, t[b][r]);
-      mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = __builtin_fmaxf(m, mx + cblk);
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-      m = m_new;
-      const float mm = m_new - cblk;
-      float psum = 0.0f;
-      uint32_t pk[2][8];
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(t[b][r] - mm);
-          const float p1 = __builtin_amdgcn_exp2f(t[b][r + 1] - mm);
-          psum += p0;
-          psum += p1;
-          pk[b][r >> 1] = pack_bf16x2(p0, p1);
-        }
-      l = l * alpha + psum;
-      if (__ballot(alpha != 1.0f) != 0) {
+  for (int st = 0; st < kStages; ++st) issue(uint32_t(st) * kStageBytes);
+  gemm::wait_vmcnt<(kStages - 1) * 4>();
+  __syncthreads();
+  load_kf(0);
+
+  auto run = [&](auto fixed_c, auto chunk_c) __attribute__((always_inline)) {
+    constexpr bool FIXED = decltype(fixed_c)::value;
+    constexpr bool CHUNK = decltype(chunk_c)::value;
+    const __bf16 b1 = __bf16(1.0f);
+    const bf16x8 ones = {b1, b1, b1, b1, b1, b1, b1, b1};
+    f32x16 lacc = {};   // FIXED: sums of the bf16 probabilities, which normalise the output
+    float psum = 0.0f;  // fp32 sums (FIXED: for lse only)
+    // Online: the running maximum; a new one rescales the output and the sum
+    auto advance = [&](float mx) __attribute__((always_inline)) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx),
+                                                       false, false);
+      mx = __builtin_fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      const float m_new = __builtin_fmaxf(m, mx);
+      if (__ballot(m_new != m) != 0) {
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        psum *= alpha;
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[mb][r] *= alpha;
       }
-      out_product(Vs, pk, o);
-
-      if (n < n_hi) store_tile(buf ^ 1);
+    };
+    // One block; EXACT: per-element bias and mask, n its number; else Jf and q the
+    // chunk's J and query columns.
+    auto step = [&](auto exact_c, int n, float Jf, const u32x4& q) __attribute__((always_inline)) {
+      constexpr bool EXACT = decltype(exact_c)::value;
+      f32x16 s[2];
+      scores(s);
+      load_vf(boff);
+      if constexpr (EXACT) {
+        exact_terms(s, n * kBKV);
+        if constexpr (!FIXED) advance(block_max(s));
+      } else {
+        if constexpr (CHUNK) add_chunk(s, Jf, q);
+        if constexpr (!FIXED) advance(block_max(s) * sc);
+      }
+      uint32_t pk[2][8];
+      float sum = 0.0f;
+      auto term = [&](int b, int r) __attribute__((always_inline)) -> float {
+        if constexpr (EXACT)
+          return s[b][r] - m;
+        else if constexpr (FIXED && CHUNK)
+          return s[b][r] * sc;  // the chunk carries -m
+        else
+          return __builtin_fmaf(s[b][r], sc, -m);
+      };
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(term(b, r));
+          const float p1 = __builtin_amdgcn_exp2f(term(b, r + 1));
+          if constexpr (!FIXED || LSE) {
+            sum += p0;
+            sum += p1;
+          }
+          pk[b][r >> 1] = pack_bf16x2(p0, p1);
+        }
+      if constexpr (!FIXED || LSE) psum += sum;
+      // the next stage landed, and every wave has read all of this one
+      gemm::wait_vmcnt<(kStages - 2) * 4>();
       __syncthreads();
+      issue(boff);
+      boff = boff + kStageBytes == kStages * kStageBytes ? 0 : boff + kStageBytes;
+      load_kf(boff);
+      // O^T += V^T . P^T over the four 16-key chunks
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const bf16x8 pf = p_chunk(pk, c);
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+          o[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c][mb], pf, o[mb], 0, 0, 0);
+        if constexpr (FIXED)
+          lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pf, lacc, 0, 0, 0);
+      }
+    };
+    using T_ = std::true_type;
+    using F_ = std::false_type;
+    const u32x4 none = {0, 0, 0, 0};
+    int n = n_lo;
+    float Jf = float(n_lo * kBKV - wq_lo);
+    for (; n < e0; ++n, Jf += float(kBKV)) step(F_{}, n, Jf, qx[1]);
+    for (; n < e1; ++n, Jf += float(kBKV)) step(T_{}, n, 0.0f, none);
+    for (; n < end; ++n, Jf += float(kBKV)) step(F_{}, n, Jf, qx[0]);
+    if (tail) {
+      // V rows past the sequence end: 0 (times a masked key's 0 probability)
+      for (int i = tid; i < (kBKV - last_rows) * 8; i += 256)
+        *reinterpret_cast<u32x4*>(ring + boff + kTileBytes + last_rows * kRowBytes + i * 16) =
+            u32x4{0, 0, 0, 0};
+      __syncthreads();
+      step(T_{}, n, 0.0f, none);
     }
-    l_tot = l + __shfl_xor(l, 32, 64);
-    l_lse = l_tot;
-  }
+    l_lse = psum + __shfl_xor(psum, 32, 64);
+    l_tot = FIXED ? lacc[0] : l_lse;
+  };
+  if (fixed && sl != 0.0f)
+    run(std::true_type{}, std::true_type{});
+  else if (fixed)
+    run(std::true_type{}, std::false_type{});
+  else if (sl != 0.0f)
+    run(std::false_type{}, std::true_type{});
+  else
+    run(std::false_type{}, std::false_type{});
+  // refills past the last block may still be landing in this workgroup's LDS
+  gemm::wait_vmcnt<0>();
 
   // normalise and store: lane holds query iq, dims 32mb + 8q + 4half + u
   if (iq < L) {
@@ -579,8 +637,13 @@ hipError_t launch_attn_fwd(const uint16_t* q, const uint16_t* k, const uint16_t*
                            const int32_t* cu_seqlens, const float* slopes, float softmax_scale,
                            float* lse, float* kmax_ws, const g5moe_attn_shape& s,
                            hipStream_t st) {
-  // key-norm bounds: block skipping (with ALiBi) and the reference-max loop
-  const bool bounds = kmax_ws != nullptr && s.total_tokens > 0;
+  // Key-norm bounds: block skipping (with ALiBi) and the reference-max loop.  The
+  // pre-pass costs a launch and a pass over k, about 4 us, which sequences of a few
+  // blocks do not earn back: with it against without, 12 heads, ALiBi 512 tokens
+  // 13.4 against 11.2 us, 2 x 1,024 20.7 against 19.6, 4,550 60 against 101; no
+  // ALiBi, 12 sequences up to 1,499 53.8 against 47.5, 2 x 2,275 49.2 against 51.8.
+  const bool bounds = kmax_ws != nullptr && s.total_tokens > 0 &&
+                      s.max_seqlen > (slopes != nullptr ? 1024 : 2048);
   const int n_kblk = int((s.total_tokens + 63) / 64);
   if (bounds) {
     hipLaunchKernelGGL(key_norm_max_kernel, dim3(unsigned(n_kblk), unsigned(s.n_kv_heads)),
@@ -612,10 +675,16 @@ hipError_t launch_attn_fwd(const uint16_t* q, const uint16_t* k, const uint16_t*
   a.total = s.total_tokens;
   const dim3 grid(unsigned((s.max_seqlen + kBQ - 1) / kBQ), unsigned(s.n_heads),
                   unsigned(s.n_seqs));
-  if (lse != nullptr)
-    hipLaunchKernelGGL(attn_fwd_kernel<true>, grid, dim3(256), 0, st, a);
+  // 64 rows of a k or v tile within 32-bit byte offsets
+  const bool wide = std::max(s.k_token_stride, s.v_token_stride) >= (int64_t(1) << 24);
+  if (wide && lse != nullptr)
+    hipLaunchKernelGGL((attn_fwd_kernel<true, true>), grid, dim3(256), 0, st, a);
+  else if (wide)
+    hipLaunchKernelGGL((attn_fwd_kernel<false, true>), grid, dim3(256), 0, st, a);
+  else if (lse != nullptr)
+    hipLaunchKernelGGL((attn_fwd_kernel<true, false>), grid, dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL(attn_fwd_kernel<false>, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_fwd_kernel<false, false>), grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
