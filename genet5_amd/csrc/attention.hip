@@ -369,67 +369,43 @@ void attn_fwd_kernel(AttnArgs a) {
   float m = fixed ? mref : -__builtin_inff(), l_tot = 0.0f, l_lse = 0.0f;
 
   // The ALiBi bias of a block wholly on one side of the wave's queries as one more
-  // 16-deep MFMA chunk, in units of raw scores: with u = sl / sc, J the block's
-  // first key from the wave's first query (a multiple of 32) and kr a key's offset
-  // in the block, the bias over sc is -+u (J + kr) +- u col (keys after / before
-  // the query), so key rows
-  //   [kr, kr, kr, Jl, Jl, Jl, Jh, Jh | Jh, 1, 1, 1, 0, 0, 0, 0]
-  // (J = Jl + Jh, Jh a multiple of 8,192: all exact in bf16 up to 2^21 keys) meet
-  // query columns [u1, u2, u3, u1, u2, u3, u1, u2 | u3, c1, c2, c3, 0, ...] of one
-  // sign, u1 + u2 + u3 and c1 + c2 + c3 bf16 splits (exact to fp32 precision; bf16
-  // products are exact in the fp32 accumulation).  The reference-max loop puts
-  // -mref / sc into c.  Per block only the J words of the key rows change.
+  // 16-deep MFMA chunk, in units of raw scores: key rows [kr, kr, kr, 1, 1, 1, 0, 0]
+  // (kr the key's offset in the block, exact in bf16; the other half zero) against
+  // query columns [-+u1, -+u2, -+u3, c1, c2, c3, 0, 0], where u1 + u2 + u3 = u =
+  // sl / sc and c1 + c2 + c3 = c = -u |j0 - i| (the reference-max loop: - mref / sc)
+  // are bf16 splits, exact to fp32 precision (bf16 products are exact in the fp32
+  // accumulation).  Per block only c's words change.
   const bool chunk_ok = __builtin_amdgcn_readfirstlane(
                             int(sc > 0.0f && sl >= 0.0f && sl < sc * 0x1p60f)) != 0;
   auto bf16r = [](float x) __attribute__((always_inline)) -> float { return float(__bf16(x)); };
-  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) -> uint32_t {
-    return pack_bf16x2(lo, hi);
-  };
-  u32x4 qx[2];            // query columns: keys after, keys before
-  uint32_t kx01[2][2];    // key words 0 and 1 of the two 32-key halves
+  const uint32_t half0 = half == 0 ? 0xffffffffu : 0u;
+  const float u = chunk_ok ? sl / sc : 0.0f;
+  const float mref_s = fixed ? mref / sc : 0.0f;
+  u32x4 kx[2];      // key rows of the two 32-key halves
+  uint32_t qu[3];   // [u1, u2], [u3, 0] and the sign bits of both (keys after: minus)
   {
-    const float u = chunk_ok ? sl / sc : 0.0f;
     const float u1 = bf16r(u), u2 = bf16r(u - u1), u3 = bf16r(u - u1 - u2);
-    const float ref = fixed ? mref / sc : 0.0f;
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const float sg = side == 0 ? -1.0f : 1.0f;
-      const float c = -sg * u * float(col) - ref;
-      const float c1 = bf16r(c), c2 = bf16r(c - c1), c3 = bf16r(c - c1 - c2);
-      const float a1 = sg * u1, a2 = sg * u2, a3 = sg * u3;
-      const u32x4 h0 = {pack2(a1, a2), pack2(a3, a1), pack2(a2, a3), pack2(a1, a2)};
-      const u32x4 h1 = {pack2(a3, c1), pack2(c2, c3), 0u, 0u};
-      qx[side] = half == 0 ? h0 : h1;
-    }
+    qu[0] = pack_bf16x2(u1, u2) & half0;
+    qu[1] = pack_bf16x2(u3, 0.0f) & half0;
+    qu[2] = 0x80008000u & half0;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const float kr = float(32 * b + col);
-      kx01[b][0] = half == 0 ? pack2(kr, kr) : pack2(0.0f, 1.0f);
-      kx01[b][1] = half == 0 ? pack2(kr, 0.0f) : pack2(1.0f, 1.0f);
+      kx[b] = u32x4{pack_bf16x2(kr, kr) & half0, pack_bf16x2(kr, 1.0f) & half0,
+                    pack_bf16x2(1.0f, 1.0f) & half0, 0u};
     }
   }
-  const uint32_t half0 = half == 0 ? 0xffffffffu : 0u;
-  const bool far = L > 8192;
-  // Adds the chunk; Jf: float(J) (its words' low bits are zero)
-  auto add_chunk = [&](f32x16* s, float Jf, const u32x4& q) __attribute__((always_inline)) {
-    uint32_t w0 = 0u, w3 = 0u;
-    float jl = Jf;
-    if (far) {
-      const float jh = __builtin_truncf(Jf * 0x1p-13f) * 0x1p13f;  // towards zero
-      jl = Jf - jh;
-      const uint32_t jb = __float_as_uint(jh);
-      w0 = (jb >> 16) & ~half0;
-      w3 = (jb | (jb >> 16)) & half0;
-    }
-    const uint32_t lb = __float_as_uint(jl);
-    const uint32_t w1 = lb & half0;
-    const uint32_t w2 = w1 | (w1 >> 16);
+  // Adds the chunk; dist = |j0 - i|, qw: the signed u words of the block's side
+  auto add_chunk = [&](f32x16* s, float dist, const uint32_t (&qw)[2])
+      __attribute__((always_inline)) {
+    const float c = -u * dist - mref_s;
+    const float c1 = bf16r(c), c2 = bf16r(c - c1), c3 = bf16r(c - c1 - c2);
+    // (the other half's key rows are zero: its query columns only have to be finite)
+    const u32x4 q = {qw[0], qw[1] | (__float_as_uint(c1) & 0xffff0000u), pack_bf16x2(c2, c3), 0u};
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const u32x4 kx = {kx01[b][0] | w0, kx01[b][1] | w1, w2, w3};
-      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kx),
+    for (int b = 0; b < 2; ++b)
+      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kx[b]),
                                                      __builtin_bit_cast(bf16x8, q), s[b], 0, 0, 0);
-    }
   };
   auto block_max = [](const f32x16* s) __attribute__((always_inline)) -> float {
     float mx = s[0][0];
@@ -488,9 +464,10 @@ void attn_fwd_kernel(AttnArgs a) {
           for (int r = 0; r < 16; ++r) o[mb][r] *= alpha;
       }
     };
-    // One block; EXACT: per-element bias and mask, n its number; else Jf and q the
-    // chunk's J and query columns.
-    auto step = [&](auto exact_c, int n, float Jf, const u32x4& q) __attribute__((always_inline)) {
+    // One block; EXACT: per-element bias and mask, n its number; else dist and qw as
+    // add_chunk takes them.
+    auto step = [&](auto exact_c, int n, float dist, const uint32_t (&qw)[2])
+        __attribute__((always_inline)) {
       constexpr bool EXACT = decltype(exact_c)::value;
       f32x16 s[2];
       scores(s);
@@ -499,7 +476,7 @@ void attn_fwd_kernel(AttnArgs a) {
         exact_terms(s, n * kBKV);
         if constexpr (!FIXED) advance(block_max(s));
       } else {
-        if constexpr (CHUNK) add_chunk(s, Jf, q);
+        if constexpr (CHUNK) add_chunk(s, dist, qw);
         if constexpr (!FIXED) advance(block_max(s) * sc);
       }
       uint32_t pk[2][8];
@@ -544,19 +521,22 @@ void attn_fwd_kernel(AttnArgs a) {
     };
     using T_ = std::true_type;
     using F_ = std::false_type;
-    const u32x4 none = {0, 0, 0, 0};
+    // the query's distance to the block's first key, exact in fp32
+    const uint32_t q_before[2] = {qu[0], qu[1]};
+    const uint32_t q_after[2] = {qu[0] ^ qu[2], qu[1] ^ (qu[2] & 0xffffu)};
     int n = n_lo;
-    float Jf = float(n_lo * kBKV - wq_lo);
-    for (; n < e0; ++n, Jf += float(kBKV)) step(F_{}, n, Jf, qx[1]);
-    for (; n < e1; ++n, Jf += float(kBKV)) step(T_{}, n, 0.0f, none);
-    for (; n < end; ++n, Jf += float(kBKV)) step(F_{}, n, Jf, qx[0]);
+    float dist = float(iq - n_lo * kBKV);
+    for (; n < e0; ++n, dist -= float(kBKV)) step(F_{}, n, dist, q_before);
+    for (; n < e1; ++n, dist -= float(kBKV)) step(T_{}, n, 0.0f, q_before);
+    dist = -dist;
+    for (; n < end; ++n, dist += float(kBKV)) step(F_{}, n, dist, q_after);
     if (tail) {
       // V rows past the sequence end: 0 (times a masked key's 0 probability)
       for (int i = tid; i < (kBKV - last_rows) * 8; i += 256)
         *reinterpret_cast<u32x4*>(ring + boff + kTileBytes + last_rows * kRowBytes + i * 16) =
             u32x4{0, 0, 0, 0};
       __syncthreads();
-      step(T_{}, n, 0.0f, none);
+      step(T_{}, n, 0.0f, q_before);
     }
     l_lse = psum + __shfl_xor(psum, 32, 64);
     l_tot = FIXED ? lacc[0] : l_lse;
@@ -638,12 +618,12 @@ hipError_t launch_attn_fwd(const uint16_t* q, const uint16_t* k, const uint16_t*
                            float* lse, float* kmax_ws, const g5moe_attn_shape& s,
                            hipStream_t st) {
   // Key-norm bounds: block skipping (with ALiBi) and the reference-max loop.  The
-  // pre-pass costs a launch and a pass over k, about 4 us, which sequences of a few
-  // blocks do not earn back: with it against without, 12 heads, ALiBi 512 tokens
-  // 13.4 against 11.2 us, 2 x 1,024 20.7 against 19.6, 4,550 60 against 101; no
-  // ALiBi, 12 sequences up to 1,499 53.8 against 47.5, 2 x 2,275 49.2 against 51.8.
+  // pre-pass costs a launch and a pass over k, about 4 us, which short sequences
+  // without ALiBi (nothing to skip) do not earn back: with it against without, 12
+  // heads, 12 sequences up to 1,499 tokens 53.8 against 47.5 us, 2 x 2,275 49.2
+  // against 51.8; with ALiBi 2 x 1,024 20.7 against 19.6, 4,550 60 against 101.
   const bool bounds = kmax_ws != nullptr && s.total_tokens > 0 &&
-                      s.max_seqlen > (slopes != nullptr ? 1024 : 2048);
+                      (slopes != nullptr || s.max_seqlen > 2048);
   const int n_kblk = int((s.total_tokens + 63) / 64);
   if (bounds) {
     hipLaunchKernelGGL(key_norm_max_kernel, dim3(unsigned(n_kblk), unsigned(s.n_kv_heads)),

@@ -595,7 +595,7 @@ g5moe_status g5moe_attn_workspace_size(const g5moe_attn_shape* shape, size_t* by
  *   softmax_lse : fp32 [n_heads, total_tokens] out (natural-log sum of the
  *   exponentials of each row, flash-attn's softmax_lse), or NULL;
  *   ws : g5moe_attn_workspace_size() bytes, or NULL.  With a workspace (and
- *   max_seqlen > 1024, or 2048 without alibi_slopes: shorter sequences do not
+ *   alibi_slopes, or max_seqlen > 2048: shorter sequences without a bias do not
  *   earn the pass back) a
  *   pre-pass writes the largest key norm of every 64-token block, and
  *   (a) with ALiBi, key blocks whose every probability is provably below 2^-64

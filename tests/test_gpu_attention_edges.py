@@ -74,8 +74,8 @@ def test_negative_slopes(cuda_device):
 
 @pytest.mark.parametrize("scale", [1.0, 3.0])
 def test_positions_past_8192(cuda_device, scale):
-    """Key offsets from the wave beyond 8,192 (the bias chunk's second offset word), both
-    loops: a nearly flat slope keeps the far keys in every row."""
+    """Long distances in the bias chunk's constant, both loops: a nearly flat slope keeps
+    the far keys in every row."""
     L = 8192 * 2 + 77
     q, k, v = inputs(L, 2, 7, cuda_device, scale)
     slopes = [1e-4, 3e-5]
