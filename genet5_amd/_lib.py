@@ -7,6 +7,7 @@ CPU or PyTorch path in its place.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from pathlib import Path
@@ -217,10 +218,9 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call `name` and raise G5MoEError on a nonzero status."""
-    L = lib()
-    st = getattr(L, name)(*args)
+    st = getattr(_lib or lib(), name)(*args)
     if st != 0:
-        msg = L.g5moe_last_error().decode(errors="replace")
+        msg = lib().g5moe_last_error().decode(errors="replace")
         raise G5MoEError(st, name, msg)
 
 
@@ -230,7 +230,24 @@ def make_shape(n_tokens: int, d_model: int, d_ff: int, n_experts: int, top_k: in
                  int(x_dtype), 0)
 
 
-def workspace_size(shape: Shape) -> int:
+@functools.lru_cache(maxsize=256)
+def _workspace_size(*fields) -> int:
     n = ctypes.c_size_t(0)
-    call("g5moe_workspace_size", ctypes.byref(shape), ctypes.byref(n))
+    call("g5moe_workspace_size", ctypes.byref(Shape(*fields)), ctypes.byref(n))
+    return int(n.value)
+
+
+def workspace_size(shape: Shape) -> int:
+    """g5moe_workspace_size: a function of the shape's fields alone."""
+    return _workspace_size(shape.n_tokens, shape.d_model, shape.d_ff, shape.n_experts,
+                           shape.top_k, shape.x_dtype, shape.reserved)
+
+
+@functools.lru_cache(maxsize=256)
+def attn_workspace_size(total_tokens: int, n_heads: int, n_kv_heads: int, head_dim: int) -> int:
+    """g5moe_attn_workspace_size, which depends on these fields alone."""
+    s = AttnShape(total_tokens=total_tokens, n_heads=n_heads, n_kv_heads=n_kv_heads,
+                  head_dim=head_dim)
+    n = ctypes.c_size_t(0)
+    call("g5moe_attn_workspace_size", ctypes.byref(s), ctypes.byref(n))
     return int(n.value)

@@ -49,6 +49,11 @@ def alibi_slopes(n_heads: int) -> List[float]:
 
 
 def _check_qkv(t: torch.Tensor, name: str, total: int, heads: int, dev: torch.device) -> None:
+    if t.device == dev and t.dtype == torch.bfloat16 and t.shape == (total, heads, HEAD_DIM):
+        st = t.stride()
+        if st[2] == 1 and st[0] % 8 == 0 and st[1] % 8 == 0 and st[0] >= 0 and st[1] >= 0 \
+                and t.data_ptr() % 16 == 0:
+            return
     if t.device != dev:
         raise ValueError(f"{name} is on {t.device}, expected {dev}")
     if t.dtype != torch.bfloat16:
@@ -106,9 +111,8 @@ def attn_varlen_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         out.stride(0), out.stride(1))
     ws = None
     if key_bounds:
-        n = ctypes.c_size_t(0)
-        _lib.call("g5moe_attn_workspace_size", ctypes.byref(shape), ctypes.byref(n))
-        ws = torch.empty(int(n.value), dtype=torch.uint8, device=dev)
+        ws = torch.empty(_lib.attn_workspace_size(T, H, Hkv, HEAD_DIM), dtype=torch.uint8,
+                         device=dev)
     _lib.call("g5moe_attn_varlen_fwd", _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(cu_seqlens),
               _ptr(alibi_slopes), ctypes.c_float(softmax_scale), _ptr(lse), _ptr(ws),
               ctypes.byref(shape), _stream(dev))
@@ -284,11 +288,15 @@ class FlashAttention(nn.Module):
         bf16 rounding of a different fp32 summation order)."""
         D = hidden_states.shape[-1]
         nq = self.num_heads * self.head_dim + 2 * self.kv_dim
+        proj = (self.q, self.k, self.v, self.o)
+        # the module's parameters; for plain projections without a walk over it
+        params = [m.weight for m in proj] if all(type(m) is nn.Linear for m in proj) \
+            else list(self.parameters())
         needs_grad = torch.is_grad_enabled() and (
-            hidden_states.requires_grad or any(p.requires_grad for p in self.parameters()))
+            hidden_states.requires_grad or any(p.requires_grad for p in params))
         return (not needs_grad and hidden_states.is_cuda
                 and hidden_states.dtype == torch.bfloat16
-                and all(p.dtype == torch.bfloat16 for p in self.parameters())
+                and all(p.dtype == torch.bfloat16 for p in params)
                 and D % 64 == 0 and D >= 128 and nq % 128 == 0 and D % 128 == 0
                 and self.num_heads * self.head_dim >= 128)
 

@@ -22,11 +22,16 @@ MAX_TOP_K = 4
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    # an address as a plain int: the bindings' argtypes convert it
+    return None if t is None else t.data_ptr()
 
 
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle on `device` (no Stream object: a short layer call
+    asks for it several times)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
 
 
 def _dtype_code(dt: torch.dtype) -> int:
@@ -38,6 +43,9 @@ def _dtype_code(dt: torch.dtype) -> int:
 
 
 def _require(t: torch.Tensor, name: str, shape, dtype, device) -> None:
+    if isinstance(t, torch.Tensor) and t.dtype == dtype and t.shape == shape and \
+            t.device == device and t.is_contiguous():
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a tensor")
     if t.device != device:
