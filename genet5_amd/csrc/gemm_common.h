@@ -41,6 +41,15 @@ __device__ __forceinline__ Offsets load_offsets(const int32_t* offsets, int n_ex
 // M0 and never keeps a value of its own there across one (clang warns that M0
 // is a reserved register, which it will not save and restore: that is not
 // needed, no caller expects M0 to survive).
+//
+// A vector-memory instruction reads a scalar register five wait states or more
+// after a VALU instruction wrote it.  The compiler keeps that rule for its own
+// loads but not inside these statements, and it reloads a spilled base with
+// v_readlane right before one.  lds_dma4_s, issued once per tile where scalar
+// registers are short, waits for all five itself (s_mov_b32 and s_nop 3).
+// lds_dma16_s, 16 times a k-step, only has M0's own wait state (a longer wait
+// costs every k-step): that no base is reloaded in front of one is checked on
+// the built library's disassembly.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));
 }
@@ -52,7 +61,7 @@ __device__ __forceinline__ void lds_dma16_s(const void* sbase, uint32_t voff, ui
                : "memory", "m0");
 }
 __device__ __forceinline__ void lds_dma4_s(const void* sbase, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1"
                :: "v"(voff), "s"(sbase), "s"(__builtin_amdgcn_readfirstlane(lds))
                : "memory", "m0");
 }
