@@ -1233,13 +1233,13 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
 }
 
 // ---------------------------------------------------------------------------
-// Ring kernel: the products with few rows (the in-place ones under small_m in the
-// launchers: a short sequence, a shard's share, a one-expert projection of one
+// Ring kernel: the products with few rows (the in-place ones that in_place_tile
+// sends here: a short sequence, a shard's share, a one-expert projection of one
 // window; the gate|up and dh products of a short sequence, ring_wide).
 //
-// With less than about one and a half 256 x 256 tiles per CU the persistent
-// kernel's workgroups each run one long tile: its k-loop waits for the two
-// stages in flight, most CUs idle, and a partial tile computes its padding rows.
+// With less than one 256 x 256 tile per CU the persistent kernel's workgroups each
+// run one long tile: its k-loop waits for the two stages in flight, many CUs idle,
+// and a partial tile computes its padding rows.
 // Here a tile is up to MAXMB 32-row blocks of one expert, exactly as many as it
 // has rows for (the expert's blocks are dealt evenly to its tiles), by 128
 // columns; the four waves take 32 columns each (for the SwiGLU modes 16 gate
@@ -1253,15 +1253,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
 // Every accumulator takes its k in the persistent kernel's order, so the outputs
 // are the same bit for bit.
 //
-// Measured against the 128 x 128 (two workgroups per CU) and 128 x 256 persistent
-// tiles that served these launches before (one GPU, captured loops, 16 experts):
-//   h . Wd^T, K = 3,072, N = 768:  96 rows 45 -> 18 us, 1,554 45 -> 21,
-//     4,096 45 -> 31-33, 9,100 51 -> 49, 18,000 95 -> 94;
-//   dGU . Wgu, K = 6,144, N = 768: 512 rows 83 -> 32, 2,200 84 -> 48,
-//     9,100 117 -> 104, 18,000 239 -> 209;
-//   one expert, K = 768: 512 x 2,304 11.9 -> 7.4, 2,048 x 2,304 13.4 -> 11.9,
-//     4,550 x 2,304 25.8 -> 23.7.
-// The gate|up and dh figures are at ring_wide.
+// The measured times are at in_place_tile and ring_wide.
 struct RingTile {
   int e, p_begin, p_end, a_row, n0;
   int mb;  // 32-row blocks of the tile; MODE 4: 0 for a tile of zero rows only
@@ -1712,12 +1704,6 @@ void launch_persist(unsigned grid, const GemmArgs& a, hipStream_t st) {
         dim3(grid), dim3(256), 0, st, a);
 }
 
-// Small M: fewer rows than one and a half 256 x 256 tiles per CU would take if
-// packed (the per-expert counts stay on the device).
-inline bool small_m(int64_t rows, int nout, unsigned ncu) {
-  return rows * nout < int64_t(3 * ncu / 2) * 256 * 256;
-}
-
 template <int MAXMB, int OCC, int MODE, bool DROP, bool PADA>
 void launch_ring_tiles(const GemmArgs& a, int64_t rows, hipStream_t st) {
   // tiles: sum_e ceil(ceil(cnt_e / 32) / MAXMB) <= rows / (32 MAXMB) + E per column,
@@ -1736,36 +1722,73 @@ inline int64_t ring_mean_blocks(int64_t rows, int n_experts) {
   return std::max<int64_t>(1, (m + 31) / 32);
 }
 
-// The ring kernel's tile height: the smallest whose tiles do not
-// outnumber the CUs, else the smallest with at most two per CU, else 128 rows.
-// Fewer rows per tile keep more CUs pulling the weight stream; a tile more than
-// the resident workgroups costs a whole tile's time (down, 4,096 rows: 432
-// 64-row tiles 33 us, 288 96-row ones 41).  128- and 96-row tiles with at most
-// one per CU take all of its LDS (OCC = 1: 26.6 against 33.5 us at 1,554 rows,
-// 96-row tiles; two stages of half the LDS leave one in flight), smaller ones
-// start sooner with half (one expert, 300 x 768 x 768: 6.2 against 6.9 us).
-template <bool PADA>
-void launch_ring(const GemmArgs& a, int64_t rows, unsigned ncu, hipStream_t st) {
-  const int64_t nb = ring_mean_blocks(rows, a.n_experts);
-  auto tiles = [&](int mb) { return (nb + mb - 1) / mb * a.n_experts * (a.Nout / 128); };
-  int mb = 1, per_cu = 1;
-  while (mb < 4 && tiles(mb) > int64_t(ncu)) ++mb;
-  if (tiles(mb) > int64_t(ncu)) {
-    per_cu = 2;
-    for (mb = 1; mb < 4 && tiles(mb) > 2 * int64_t(ncu);) ++mb;
+// Tiles of h rows that experts of the mean row count take under uniform routing: the
+// sum of P(count > j h) for normal counts (mean and variance `mean`), m / h + 1/2
+// where they spread over several heights.  One expert's count is the row count.
+inline double expected_m_tiles(double mean, int n_experts, int h) {
+  if (n_experts == 1) return std::ceil(mean / h);
+  const double sd = std::sqrt(mean);
+  if (2.0 * sd > h) return n_experts * (mean / h + 0.5);
+  double j = std::max(0.0, std::floor((mean - 4.0 * sd) / h)), sum = j;
+  for (; j * h < mean + 4.0 * sd; j += 1.0)  // (8 sd <= 4 h: a few steps)
+    sum += 0.5 * std::erfc((j * h + 0.5 - mean) / (sd * 1.4142135623730951));
+  return n_experts * sum;
+}
+
+// The tile of an in-place product (MODE 0): the ring kernel's 32 mb rows by 128
+// columns, or (mb = 0) the persistent kernel's 256 x 256 (256 x 128 where Nout is no
+// multiple of 256), by the time their expected tiles take.  The costs below are
+// measured microseconds per k-step of one round of resident tiles, weights from HBM
+// (kernel traces of whole layer calls and of single products over rotating weights;
+// 16 and 8 experts, K = 1,024-6,144; one expert, K = 768-3,072): ring tiles at most
+// one per CU, just above one, two per CU; of a ring round that follows a full one
+// two thirds where it has at most one tile per CU; a persistent round, 0.8 of one
+// for a remainder that runs as halves.  One deviation of the tile count is added:
+// a tile too many costs a round.  128- and 96-row tiles with at most one per CU take
+// all of its LDS (occ = 1: 38 against 51 us at 2,048 tokens; two stages of half the
+// LDS leave one in flight), smaller ones start as soon with half.
+// Measured, us (this rule's choice; two-per-CU 128 x 128 persistent tiles, or 128 x
+// 256 for dX, that served these launches before; ring tiles at every size), 16
+// experts, d = 768, F = 3,072, tokens (2 rows each):
+//   down  300 24.7 42.0 24.7   777 29.2 42.4 38.1   1,100 30.6 42.5 30.6
+//         2,048 38.5 44.6 47.5   3,000 57 59 57   4,550 63.5 60.8 63.5
+//         6,000 75 87 104   8,000 78 104 112   13,000 128 143 167   16,000 148 178 204
+//   dX    1,100 64 136 64   2,048 75 138 92   4,550 123 142 123
+//         6,000 138 242 201   8,000 145 254 214   16,000 289 490 411
+//   one expert, K = 768: 512 x 2,304 8.1 14.7 8.1, 4,550 x 2,304 21.3 26.2 23.7,
+//         12,000 x 768 19.9 25.7 23.0.
+// 96-row tiles beyond one per CU are left out: 128-row ones take as long there.
+struct InPlaceTile {
+  int mb;   // 32-row blocks of a ring tile; 0: persistent
+  int occ;  // ring workgroups per CU
+};
+inline InPlaceTile in_place_tile(int64_t rows, const GemmArgs& a, unsigned ncu) {
+  static constexpr double kRing[4][3] = {
+      {0.50, 0.74, 0.84}, {0.60, 0.90, 0.99}, {0.65, 0.65, 0.65}, {0.78, 1.04, 1.32}};
+  const double mean = double(rows) / a.n_experts, cu = double(ncu);
+  const double spread = a.n_experts > 1 ? 0.5 * std::sqrt(double(a.n_experts)) : 0.0;
+  const bool n256 = a.Nout % 256 == 0;
+  // (k-step counts that are no multiple of 3 run two fragment slots)
+  const double step = !n256 ? 1.02 : (a.K / 64 % 3 == 0 ? 1.45 : 1.9);
+  const double pt = (expected_m_tiles(mean, a.n_experts, 256) + spread) *
+                    (a.Nout / (n256 ? 256 : 128));
+  const double q = std::floor(pt / cu), r = pt - q * cu;
+  double best = step * (q + (r < 1.0 ? 0.0 : (n256 && q > 0.0 && 2.0 * r <= cu ? 0.8 : 1.0)));
+  InPlaceTile tile{0, 1};
+  for (int mb = 1; mb <= 4; ++mb) {
+    const double* c = kRing[mb - 1];
+    const double t = (expected_m_tiles(mean, a.n_experts, 32 * mb) + spread) * (a.Nout / 128);
+    if (mb == 3 && t > cu) continue;
+    const double full = std::floor(t / (2.0 * cu)), rem = t - full * 2.0 * cu;
+    const double cost = t <= cu         ? c[0]
+                        : t <= 2.0 * cu ? c[1] + (c[2] - c[1]) * (t / cu - 1.0)
+                                        : c[2] * (full + (rem < 1.0 ? 0.0 : rem <= cu ? 0.66 : 1.0));
+    if (cost < best) {
+      best = cost;
+      tile = InPlaceTile{mb, t <= cu && mb > 2 ? 1 : 2};
+    }
   }
-  if (mb == 1)
-    launch_ring_tiles<1, 2, 0, false, PADA>(a, rows, st);
-  else if (mb == 2)
-    launch_ring_tiles<2, 2, 0, false, PADA>(a, rows, st);
-  else if (mb == 3 && per_cu == 1)
-    launch_ring_tiles<3, 1, 0, false, PADA>(a, rows, st);
-  else if (mb == 3)
-    launch_ring_tiles<3, 2, 0, false, PADA>(a, rows, st);
-  else if (per_cu == 1)
-    launch_ring_tiles<4, 1, 0, false, PADA>(a, rows, st);
-  else
-    launch_ring_tiles<4, 2, 0, false, PADA>(a, rows, st);
+  return tile;
 }
 
 // Whether a gate|up (MODE 1 / 5) or dh (MODE 4) launch takes the ring kernel: its
@@ -1966,8 +1989,17 @@ namespace {
 template <bool PADA>
 hipError_t launch_in_place(const GemmArgs& a, int64_t rows, hipStream_t st) {
   const unsigned ncu = unsigned(device_cu_count());
-  if (small_m(rows, a.Nout, ncu)) {
-    launch_ring<PADA>(a, rows, ncu, st);
+  const InPlaceTile t = in_place_tile(rows, a, ncu);
+  if (t.mb == 1) {
+    launch_ring_tiles<1, 2, 0, false, PADA>(a, rows, st);
+  } else if (t.mb == 2) {
+    launch_ring_tiles<2, 2, 0, false, PADA>(a, rows, st);
+  } else if (t.mb == 3) {
+    launch_ring_tiles<3, 1, 0, false, PADA>(a, rows, st);
+  } else if (t.mb == 4 && t.occ == 1) {
+    launch_ring_tiles<4, 1, 0, false, PADA>(a, rows, st);
+  } else if (t.mb == 4) {
+    launch_ring_tiles<4, 2, 0, false, PADA>(a, rows, st);
   } else if (a.Nout % 256 == 0) {
     const unsigned grid = std::min(grid_bound<256, 256>(rows, a.n_experts, a.Nout), ncu);
     launch_persist<256, 256, G5_DN_BK, G5_DN_STAGES, G5_DN_GM, 0, true, false, PADA>(grid, a, st);

@@ -19,14 +19,21 @@ def _offsets(counts, dev):
     return off, torch.tensor(off, dtype=torch.int32, device=dev)
 
 
+# The tile that the launch takes on 256 CUs (blocks of 32 rows, workgroups per CU) stands
+# after each case: every form of the kernel has one.
 @pytest.mark.parametrize("K,n_out,counts", [
-    (128, 128, [1, 0, 31, 32, 33]),                    # the smallest: two k-steps, one n-tile
-    (192, 256, [0, 5, 64, 65]),                        # odd k-step count
-    (768, 768, [6, 0, 9, 4, 1, 12, 7, 0]),             # one block per tile
-    (3072, 768, [97, 96, 0, 128, 31, 64, 65, 129, 1, 95, 100, 90, 97, 97, 97]),
-    (1024, 768, [257, 255, 256, 288, 289, 1, 0, 320]),  # three- and four-block tiles
-    (768, 384, [1137]),                                # one expert, an odd number of n-tiles
-    (256, 2304, [4550]),
+    (128, 128, [1, 0, 31, 32, 33]),         # 1, two: the smallest, two k-steps, one n-tile
+    (192, 256, [0, 5, 64, 65]),             # 1, two: odd k-step count
+    (768, 768, [6, 0, 9, 4, 1, 12, 7, 0]),  # 1, two
+    (3072, 768, [97, 96, 0, 128, 31, 64, 65, 129, 1, 95, 100, 90, 97, 97, 97]),  # 2, two
+    (1024, 768, [257, 255, 256, 288, 289, 1, 0, 320]),  # 2, two
+    (768, 384, [1137]),                     # 1, two: one expert, an odd number of n-tiles
+    (256, 2304, [4550]),                    # persistent: one expert in the larger launch too
+    (192, 768, [137, 96, 97, 0, 128, 129, 192, 193, 31, 160, 161, 95, 288, 289, 33]),  # 3, one
+    (3072, 768, [137, 96, 97, 0, 128, 129, 192, 193, 31, 160, 161, 95, 288, 289, 33]),  # 3, one
+    (256, 768, [256, 255, 257, 0, 1, 128, 129, 300, 511, 512, 385, 320, 290, 230, 270]),  # 4, one
+    (128, 768, [375, 384, 385, 0, 31, 33, 512, 513, 400, 390, 700, 640, 641, 128, 129]),  # 4, two
+    (768, 2304, [2048]),                    # 4, two: one expert
 ])
 @pytest.mark.parametrize("packed", [False, True])
 def test_ring_equals_persistent_tiles(cuda_device, K, n_out, counts, packed):
