@@ -138,8 +138,9 @@ __device__ __forceinline__ void lds_dma16_v(const char* addr, uint32_t lds) {
 #pragma clang diagnostic pop
 
 // LSE: softmax_lse is written (a.lse != nullptr).  WIDE: a token stride of k or v
-// too large for 32-bit offsets inside a 64-key tile.
-template <bool LSE, bool WIDE>
+// too large for 32-bit offsets inside a 64-key tile.  NEG: a negative scale, taken as
+// its magnitude on negated queries (exactly the same products).
+template <bool LSE, bool WIDE, bool NEG>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
 void attn_fwd_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char ring[kStages * kStageBytes];
@@ -164,7 +165,7 @@ void attn_fwd_kernel(AttnArgs a) {
   const int wq_lo = q0 + wave * 32;          // the wave's query range
   const int wq_hi = wq_lo + 31;
   const float sl = a.slopes != nullptr ? a.slopes[hq] * kLog2e : 0.0f;
-  const float sc = a.sc;
+  const float sc = NEG ? -a.sc : a.sc;
 
   // Q^T operand: lane holds query iq, head dims 16kc + 8*half .. +8.
   bf16x8 qf[4];
@@ -181,6 +182,10 @@ void attn_fwd_kernel(AttnArgs a) {
 #pragma unroll
     for (int kc = 0; kc < 4; ++kc) {
       u32x4 w = __builtin_bit_cast(u32x4, qf[kc]);
+      if constexpr (NEG) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] ^= 0x80008000u;
+      }
       asm volatile("" : "+v"(w));
       qf[kc] = __builtin_bit_cast(bf16x8, w);
     }
@@ -235,7 +240,7 @@ void attn_fwd_kernel(AttnArgs a) {
     // bound is the same in every lane (red); false for inf / NaN.  sl < 2^60 sc
     // keeps the slope in units of raw scores (u = sl / sc) and its products
     // with key offsets and distances (< 2^31) finite.
-    fixed = __builtin_amdgcn_readfirstlane(int(sc > 0.0f && sl >= 0.0f && sl < sc * 0x1p60f &&
+    fixed = __builtin_amdgcn_readfirstlane(int(!NEG && sc > 0.0f && sl >= 0.0f && sl < sc * 0x1p60f &&
                                                2.0f * bound <= kFixedGap)) != 0;
     mref = sc * __builtin_sqrtf(ss_own) * kmx;
   }
@@ -374,9 +379,12 @@ void attn_fwd_kernel(AttnArgs a) {
   // query columns [-+u1, -+u2, -+u3, c1, c2, c3, 0, 0], where u1 + u2 + u3 = u =
   // sl / sc and c1 + c2 + c3 = c = -u |j0 - i| (the reference-max loop: - mref / sc)
   // are bf16 splits, exact to fp32 precision (bf16 products are exact in the fp32
-  // accumulation).  Per block only c's words change.
+  // accumulation).  Per block only c's words change.  Slopes and scales of either sign
+  // take it; a scale of 0 or a slope out of range makes every block exact (8 x 4,550
+  // tokens, 12 heads, this against every block exact: ALiBi's slopes times -0.01 679
+  // against 790 us, a scale of -0.125 without a bias 656 against 792).
   const bool chunk_ok = __builtin_amdgcn_readfirstlane(
-                            int(sc > 0.0f && sl >= 0.0f && sl < sc * 0x1p60f)) != 0;
+                            int(sc > 0.0f && __builtin_fabsf(sl) < sc * 0x1p60f)) != 0;
   auto bf16r = [](float x) __attribute__((always_inline)) -> float { return float(__bf16(x)); };
   const uint32_t half0 = half == 0 ? 0xffffffffu : 0u;
   const float u = chunk_ok ? sl / sc : 0.0f;
@@ -657,14 +665,17 @@ hipError_t launch_attn_fwd(const uint16_t* q, const uint16_t* k, const uint16_t*
                   unsigned(s.n_seqs));
   // 64 rows of a k or v tile within 32-bit byte offsets
   const bool wide = std::max(s.k_token_stride, s.v_token_stride) >= (int64_t(1) << 24);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, a); };
+  const bool neg = softmax_scale < 0.0f;
   if (wide && lse != nullptr)
-    hipLaunchKernelGGL((attn_fwd_kernel<true, true>), grid, dim3(256), 0, st, a);
+    neg ? launch(attn_fwd_kernel<true, true, true>) : launch(attn_fwd_kernel<true, true, false>);
   else if (wide)
-    hipLaunchKernelGGL((attn_fwd_kernel<false, true>), grid, dim3(256), 0, st, a);
+    neg ? launch(attn_fwd_kernel<false, true, true>) : launch(attn_fwd_kernel<false, true, false>);
   else if (lse != nullptr)
-    hipLaunchKernelGGL((attn_fwd_kernel<true, false>), grid, dim3(256), 0, st, a);
+    neg ? launch(attn_fwd_kernel<true, false, true>) : launch(attn_fwd_kernel<true, false, false>);
   else
-    hipLaunchKernelGGL((attn_fwd_kernel<false, false>), grid, dim3(256), 0, st, a);
+    neg ? launch(attn_fwd_kernel<false, false, true>)
+        : launch(attn_fwd_kernel<false, false, false>);
   return hipGetLastError();
 }
 

@@ -46,8 +46,8 @@ def check(got, ref, what):
 @pytest.mark.parametrize("softmax_scale", [0.125, 0.5, 0.0, -0.125])
 def test_block_edges(cuda_device, use_alibi, softmax_scale):
     """Lengths around the 32-query, 64-key and 128-query edges, in one packed call, with
-    scales that the fast path takes and ones (zero, negative) that only the exact path
-    does."""
+    scales that the fast path takes (a negative one on negated queries) and one, zero, that
+    only the exact path does."""
     lens = [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 257]
     cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
     q, k, v = inputs(cu[-1], 4, 3, cuda_device)
@@ -70,6 +70,20 @@ def test_negative_slopes(cuda_device):
                                     200, 0.125, torch.tensor(slopes, device=cuda_device))
     torch.cuda.synchronize()
     check(out, reference(q, k, v, cu, 0.125, slopes), "negative slope")
+
+
+@pytest.mark.parametrize("softmax_scale", [0.125, -0.125, 0.0])
+@pytest.mark.parametrize("slopes", [[-0.02, -0.3, 0.3, -1e-4], [0.0, -5.0, 1e30, -1e30]])
+def test_slopes_of_either_sign_over_many_blocks(cuda_device, slopes, softmax_scale):
+    """Whole blocks before and after the queries with a bias that grows with the distance,
+    and slopes that leave the bias chunk's range (2^60 scale), where the exact path serves."""
+    cu = [0, 700, 829]
+    q, k, v = inputs(cu[-1], 4, 13, cuda_device)
+    print(f"slopes {slopes} scale {softmax_scale}", flush=True)
+    out = attention.attn_varlen_fwd(q, k, v, torch.tensor(cu, dtype=torch.int32, device=cuda_device),
+                                    700, softmax_scale, torch.tensor(slopes, device=cuda_device))
+    torch.cuda.synchronize()
+    check(out, reference(q, k, v, cu, softmax_scale, slopes), f"{slopes} {softmax_scale}")
 
 
 @pytest.mark.parametrize("scale", [1.0, 3.0])
