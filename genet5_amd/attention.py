@@ -289,14 +289,16 @@ class FlashAttention(nn.Module):
         D = hidden_states.shape[-1]
         nq = self.num_heads * self.head_dim + 2 * self.kv_dim
         proj = (self.q, self.k, self.v, self.o)
-        # the module's parameters; for plain projections without a walk over it
-        params = [m.weight for m in proj] if all(type(m) is nn.Linear for m in proj) \
-            else list(self.parameters())
+        # the fused products know a weight and nothing else: a replaced projection (a
+        # bias, an adapter) keeps its own forward
+        if not all(type(m) is nn.Linear and m.bias is None for m in proj):
+            return False
+        weights = [m.weight for m in proj]
         needs_grad = torch.is_grad_enabled() and (
-            hidden_states.requires_grad or any(p.requires_grad for p in params))
+            hidden_states.requires_grad or any(w.requires_grad for w in weights))
         return (not needs_grad and hidden_states.is_cuda
                 and hidden_states.dtype == torch.bfloat16
-                and all(p.dtype == torch.bfloat16 for p in params)
+                and all(w.dtype == torch.bfloat16 for w in weights)
                 and D % 64 == 0 and D >= 128 and nq % 128 == 0 and D % 128 == 0
                 and self.num_heads * self.head_dim >= 128)
 

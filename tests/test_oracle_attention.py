@@ -203,3 +203,41 @@ def test_attn_wrappers_refuse_cpu_and_unsupported_modes():
         attention.flash_attn_varlen_func(q, q, q, cu, cu, 4, 4, causal=True)
     with pytest.raises(NotImplementedError, match="head_dim"):
         attention.FlashAttention(attention.FlashAttentionConfig(embed_dim=768, num_heads=6))
+
+
+def test_module_fuses_only_plain_projections():
+    """The fused inference projections multiply by the weights alone, so a projection that a
+    caller replaced (a bias, a wrapper) keeps its own forward, whatever needs a gradient."""
+    from types import SimpleNamespace
+
+    import torch
+    import torch.nn as nn
+
+    from genet5_amd import attention
+    cfg = attention.FlashAttentionConfig(embed_dim=256, num_heads=4)
+    make = lambda: attention.FlashAttention(cfg).to(torch.bfloat16).requires_grad_(False).eval()
+    # (what the choice looks at of a GPU input)
+    x = SimpleNamespace(shape=(1, 8, 256), dtype=torch.bfloat16, is_cuda=True, requires_grad=False)
+    m = make()
+    assert m._fused_projections(x)
+    m.q.weight.requires_grad_(True)
+    assert not m._fused_projections(x)
+    with torch.no_grad():
+        assert m._fused_projections(x)
+    for name in "qkvo":
+        for grad in (False, True):
+            m = make()
+            biased = nn.Linear(256, 256).to(torch.bfloat16).requires_grad_(False)
+            biased.bias.requires_grad_(grad)
+            setattr(m, name, biased)
+            assert not m._fused_projections(x)
+            with torch.no_grad():
+                assert not m._fused_projections(x)
+
+    class Wrapped(nn.Linear):
+        def forward(self, t):
+            return 2 * super().forward(t)
+
+    m = make()
+    m.v = Wrapped(256, 256, bias=False).to(torch.bfloat16).requires_grad_(False)
+    assert not m._fused_projections(x)
