@@ -125,3 +125,18 @@ def test_attention_backend_choice_is_explicit():
     m = m.to(torch.bfloat16)
     assert m.layers[0].self_attn.slopes.dtype == torch.float32
     assert m.layers[0].self_attn.slopes[1].item() == 2.0 ** -8
+
+
+def test_stream_handle_without_torchs_private_name(monkeypatch):
+    """The bindings ask torch for the current stream's raw handle, by its private name where
+    torch has it, else through the public interface."""
+    from types import SimpleNamespace
+
+    from genet5_amd import ops
+    dev = torch.device("cuda", 3)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda d: SimpleNamespace(cuda_stream=1000 + d.index))
+    monkeypatch.setattr(ops, "_raw_stream", lambda index: 10 + index)
+    assert ops._stream(dev) == 13
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream(dev) == 1003
