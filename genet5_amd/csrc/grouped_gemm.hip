@@ -1866,6 +1866,8 @@ hipError_t launch_gate_up(const uint16_t* xb, const int32_t* perm, const int32_t
   a.ldc = s.d_ff;
   a.ldc2 = 2 * s.d_ff;
   if (a.K < G5_GU_STAGES * G5_GU_BK) return hipErrorInvalidValue;
+  const bool dropout = drop != nullptr && drop->on;
+  if (dropout && gu == nullptr) return hipErrorInvalidValue;  // a training-forward mode
   int nb = 0;
   if (gu == nullptr && ring_wide(a, nk, 4, unsigned(device_cu_count()), &nb)) {
     launch_ring_wide<1, false, false>(a, nk, nb, st);
@@ -1876,10 +1878,8 @@ hipError_t launch_gate_up(const uint16_t* xb, const int32_t* perm, const int32_t
   const unsigned grid = bm192 ? grid_bound<192, 256>(nk, s.n_experts, a.Nout)
                               : grid_bound<256, 256>(nk, s.n_experts, a.Nout);
   const unsigned pgrid = std::min<unsigned>(grid, unsigned(device_cu_count()));
-  const bool dropout = drop != nullptr && drop->on;
   a.xs = xcd_split(gu != nullptr ? (dropout ? 3 : 2) : (bm192 ? 1 : 0), pgrid, a.K, a.Nout, st);
   if (dropout) {
-    if (gu == nullptr) return hipErrorInvalidValue;  // dropout is a training-forward mode
     a.drop_seed_lo = drop->seed_lo;
     a.drop_seed_hi = drop->seed_hi;
     a.drop_thr = drop->thr;
