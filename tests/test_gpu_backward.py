@@ -510,50 +510,71 @@ def test_gate_up_train_factors(cuda_device, n, d, F, E, k, p):
         assert np.all(got[m == 0] == 0), name
 
 
+def _check_dh_swiglu(dev, counts, F, packed):
+    import ctypes
+    from genet5_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(3)
+    E, d, k = len(counts), 768, 2
+    offsets = np.zeros(E + 1, np.int32)
+    offsets[1:] = np.cumsum(counts)
+    T = int(offsets[-1])
+    t_off = torch.tensor(offsets, dtype=torch.int32, device=dev)
+    wrows = [max(384, 192 * -(-c // 192)) for c in counts]
+    kmax = 0 if packed else ops.wgrad_kmax(max(counts))
+    prows = ops.packed_rows(T, E) if packed else E * kmax
+    starts = [sum(wrows[:e]) if packed else e * kmax for e in range(E)]
+    dy = torch.randn(T + ops.ROW_PAD, d, device=dev, generator=g).to(torch.bfloat16)
+    dy_buf = torch.zeros(prows + ops.ROW_PAD, d, dtype=torch.bfloat16, device=dev)
+    for e, c in enumerate(counts):
+        dy_buf[starts[e]:starts[e] + c] = dy[offsets[e]:offsets[e + 1]]
+    wd_t = (torch.randn(E, F, d, device=dev, generator=g) * 0.05).to(torch.bfloat16)
+    fac = torch.randn(T, 2 * F, device=dev, generator=g).to(torch.bfloat16)
+    dgu = torch.full((prows + ops.ROW_PAD, 2 * F), -7.0, dtype=torch.bfloat16, device=dev)
+    n_tok = (T + k - 1) // k
+    shape = _lib.make_shape(n_tok, d, F, E, k, _lib.DTYPE_BF16)
+    print(f"  dh swiglu counts={counts} F={F} kmax={kmax}", flush=True)
+    _lib.call("g5moe_dh_swiglu_backward", ops._ptr(dy_buf), kmax, ops._ptr(t_off),
+              ops._ptr(wd_t), ops._ptr(fac), ops._ptr(dgu), ctypes.byref(shape),
+              ops._stream(dev))
+    dh = ops.grouped_gemm_padded(dy_buf, kmax, T, t_off, wd_t)  # [T, F] bf16
+    torch.cuda.synchronize()
+    end = 0
+    for e, c in enumerate(counts):
+        o0, s0 = int(offsets[e]), starts[e]
+        a, b = _split_packed(fac[o0:o0 + c], F)
+        dhe = dh[o0:o0 + c].float()
+        ref = torch.stack([(dhe * a.float()).to(torch.bfloat16).view(c, F // 32, 32),
+                           (dhe * b.float()).to(torch.bfloat16).view(c, F // 32, 32)],
+                          2).reshape(c, 2 * F)
+        assert torch.equal(dgu[s0:s0 + c], ref), e
+        assert not dgu[s0 + c:s0 + wrows[e]].any(), e
+        assert (dgu[end:s0] == -7.0).all(), e
+        end = s0 + wrows[e]
+    assert (dgu[end:] == -7.0).all()
+
+
 @pytest.mark.parametrize("counts", [[0, 1, 192, 255, 256, 385, 2000, 4100], [700, 3, 0, 0]])
 def test_dh_swiglu_fused_equals_staged(cuda_device, counts):
     """g5moe_dh_swiglu_backward against the staged computation: dh from
     g5moe_grouped_gemm_padded (the same product, stored bf16), times the factors in
     fp32 with one bf16 rounding (torch) — bit for bit in every expert's rows, zeros
-    in the rows up to the weight gradient's row count, rows past it untouched."""
-    import ctypes
-    from genet5_amd import _lib
-    dev = cuda_device
-    g = torch.Generator(device=dev).manual_seed(3)
-    E, d, F, k = len(counts), 768, 512, 2
-    offsets = np.zeros(E + 1, np.int32)
-    offsets[1:] = np.cumsum(counts)
-    T = int(offsets[-1])
-    t_off = torch.tensor(offsets, dtype=torch.int32, device=dev)
-    kmax = ops.wgrad_kmax(max(counts))
-    dy = torch.randn(T + ops.ROW_PAD, d, device=dev, generator=g).to(torch.bfloat16)
-    dy_buf = torch.zeros(E * kmax + ops.ROW_PAD, d, dtype=torch.bfloat16, device=dev)
-    dy_buf[:E * kmax] = ops.pad_rows(dy, None, t_off, E, kmax, k).view(E * kmax, d)
-    wd_t = (torch.randn(E, F, d, device=dev, generator=g) * 0.05).to(torch.bfloat16)
-    fac = torch.randn(T, 2 * F, device=dev, generator=g).to(torch.bfloat16)
-    sentinel = torch.full((E * kmax + ops.ROW_PAD, 2 * F), -7.0, dtype=torch.bfloat16,
-                          device=dev)
-    dgu = sentinel.clone()
-    n_tok = (T + k - 1) // k
-    shape = _lib.make_shape(n_tok, d, F, E, k, _lib.DTYPE_BF16)
-    print(f"  counts={counts} kmax={kmax}", flush=True)
-    _lib.call("g5moe_dh_swiglu_backward", ops._ptr(dy_buf), kmax, ops._ptr(t_off),
-              ops._ptr(wd_t), ops._ptr(fac), ops._ptr(dgu), ctypes.byref(shape),
-              ops._stream(dev))
-    dh = ops.grouped_gemm_padded(dy_buf, kmax, T, t_off, wd_t)  # [T, F] bf16
-    a, b = _split_packed(fac, F)
-    dg = (dh.float() * a.float()).to(torch.bfloat16)
-    du = (dh.float() * b.float()).to(torch.bfloat16)
-    ref = torch.stack([dg.view(T, F // 32, 32), du.view(T, F // 32, 32)], 2).reshape(T, 2 * F)
-    torch.cuda.synchronize()
-    for e, c in enumerate(counts):
-        o0 = int(offsets[e])
-        kr = max(384, 192 * -(-c // 192))
-        rows = dgu[e * kmax: e * kmax + kmax]
-        assert torch.equal(rows[:c], ref[o0:o0 + c]), e
-        assert not rows[c:kr].any(), e
-        assert torch.equal(rows[kr:], sentinel[:kmax - kr]), e
-    assert torch.equal(dgu[E * kmax:], sentinel[E * kmax:])
+    in the rows up to the weight gradient's row count, rows past it untouched.  (F =
+    512: so few n-tiles that the ring kernel takes them.)"""
+    _check_dh_swiglu(cuda_device, counts, 512, packed=False)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("counts", [
+    # about 340 rows per expert: one to two tiles per workgroup, n-half remainders
+    [0, 1, 255, 257, 256, 384, 385, 383, 193, 700, 1100, 3, 512, 513, 640, 900],
+    # six or seven tiles per workgroup, one expert with over a third of the rows
+    [0, 1, 255, 257, 12000, 9001, 4000, 2304, 511, 0, 1, 767, 1025, 900, 31, 33],
+])
+def test_dh_swiglu_persistent_equals_staged(cuda_device, counts, packed):
+    """The same on the persistent tiles (F = 3,072 and more than about 226 rows per expert,
+    past the ring kernel's rule): stage buffers refilled across tiles, half tiles, partial
+    last tiles and the zero rows after them, in both padded layouts."""
+    _check_dh_swiglu(cuda_device, counts, 3072, packed)
 
 
 @pytest.mark.parametrize("n,d,E,k", [(36400, 768, 16, 2), (4097, 768, 16, 2), (1, 768, 16, 2),

@@ -1,19 +1,17 @@
-"""The persistent grouped GEMM (g5moe_grouped_gemm, the kernel of the down product
-and the backward's dh / dX products) across its pipeline variants: two fragment
-slots (k-steps not a multiple of 3), three slots with the third A stage in the
-epilogue region (k-steps a multiple of 3, at least 6), 128- and 256-column tiles,
-the n-half tail, 128-row tiles (launches whose rows give fewer than 1.5 full
-256 x 256 tiles per CU), experts with no rows, partial last tiles and workgroups
-that run many tiles in a row.
+"""The grouped GEMM (g5moe_grouped_gemm, the kernels of the down product and the
+backward's dh / dX products) across its persistent kernel's pipeline variants: two
+fragment slots (k-steps not a multiple of 3), three slots with the third A stage in the
+epilogue region (k-steps a multiple of 3, at least 6), 128- and 256-column tiles, the
+n-half tail, experts with no rows, partial last tiles and workgroups that run many tiles
+in a row; and its ring kernel, which serves the launches with few rows.
 
 Two checks per case.  (1) Each expert launched alone gives the same bits as the
 full launch: an output element's MFMA chain runs over k in one fixed order whatever
 workgroup, tile slot, stage buffer or tile height computes it, so a stage that lands
-in the wrong buffer, a stale refill or a skipped tile breaks equality (a small
-expert's solo launch takes 128-row tiles where the full launch may take 256-row
-ones).  (2) Every expert's rows
-match a float32 torch product of the same bf16 operands (rtol = atol = 2e-2 on
-unit-scale outputs)."""
+in the wrong buffer, a stale refill or a skipped tile breaks equality (the small experts'
+solo launches take ring tiles where the full launch takes the persistent ones).  (2) Every
+expert's rows match a float32 torch product of the same bf16 operands (rtol = atol = 2e-2
+on unit-scale outputs)."""
 import numpy as np
 import pytest
 import torch
@@ -29,14 +27,21 @@ def _offsets(counts, device):
     return off, torch.tensor(off, dtype=torch.int32, device=device)
 
 
+# The full launch's tile on 256 CUs stands after each case; experts of a few thousand rows
+# and fewer run ring tiles alone.
 @pytest.mark.parametrize("K,n_out,counts", [
-    (384, 256, [40000, 0, 257, 9000]),         # nk = 6: shortest three-stage tile
-    (384, 256, [100000, 0, 257, 9000]),        # 256-row tiles, solos of 257 / 9000: 128
-    (576, 768, [0, 1, 255, 256, 4097, 30000]),  # nk = 9, three n-tiles, half tail
-    (448, 256, [12000, 3, 700]),               # nk = 7: two fragment slots
-    (128, 128, [5000, 0, 999]),                # nk = 2, 128-column tiles
-    (3072, 768, [9000, 4551, 0, 311]),         # the down product's K
-    (6144, 768, [2500, 1300]),                 # the dX product's K
+    (384, 256, [40000, 0, 257, 9000]),         # persistent; nk = 6: shortest three-stage tile
+    (384, 256, [100000, 0, 257, 9000]),        # persistent, more tiles per workgroup
+    (576, 768, [0, 1, 255, 256, 4097, 30000]),  # persistent; nk = 9, three n-tiles, half tail
+    (448, 256, [12000, 3, 700]),               # ring; nk = 7
+    (448, 256, [50000, 3, 700]),               # persistent; nk = 7: two fragment slots
+    (128, 128, [5000, 0, 999]),                # ring; nk = 2
+    (128, 128, [60000, 0, 999]),               # persistent, 128-column tiles; nk = 2
+    (768, 384, [30000, 257, 0, 31]),           # persistent, 128-column tiles, three slots
+    (512, 384, [30000, 257, 0, 31]),           # persistent, 128-column tiles, two slots
+    (3072, 768, [9000, 4551, 0, 311]),         # persistent; the down product's K
+    (6144, 768, [2500, 1300]),                 # ring; the dX product's K
+    (6144, 768, [14000, 1300, 0, 97]),         # persistent; the dX product's K
 ])
 def test_grouped_gemm_pipeline_variants(cuda_device, K, n_out, counts):
     print(f"case K={K} n_out={n_out} counts={counts}", flush=True)
@@ -67,19 +72,19 @@ def test_grouped_gemm_pipeline_variants(cuda_device, K, n_out, counts):
     (256, [569, 0, 4000, 1, 255, 256, 257, 1700]),
     (768, [4550, 4550]),                                   # the EP-8 shard: 2 experts
 ])
-def test_small_m_down_two_per_cu_equals_grouped_gemm(cuda_device, d, counts):
-    """The down product at small M (a DP-8 / EP-8 shard's rows) runs 128 x 128 tiles
-    with two workgroups per CU (g5moe_expert_down), while g5moe_grouped_gemm takes
-    one 128 x 256 workgroup per CU there: each output's MFMA chain runs over k in
-    the same order whatever the tile shape, so y_perm must equal the grouped GEMM
-    on the same h and w_down bit for bit, with empty experts and partial tiles."""
+def test_down_of_few_rows_equals_a_larger_launch(cuda_device, d, counts):
+    """The down product (g5moe_expert_down) of a DP-8 / EP-8 shard's rows runs ring tiles;
+    the same experts beside one of 48,000 rows run the persistent 256 x 256 tiles
+    (g5moe_grouped_gemm, at most eight of them per launch).  Each output's MFMA chain runs
+    over k in the same order whatever the tile, so y_perm must equal the larger launches'
+    rows bit for bit, with empty experts and partial tiles."""
     import ctypes
     from genet5_amd import _lib
-    F, k = 3072, 2
+    F, k, big = 3072, 2, 48000
     E = len(counts)
     rows = int(sum(counts))
     assert rows % k == 0
-    print(f"small-M down d={d} E={E} rows={rows}", flush=True)
+    print(f"down d={d} E={E} rows={rows}", flush=True)
     g = torch.Generator(device=cuda_device).manual_seed(rows + d)
     off, t_off = _offsets(counts, cuda_device)
     shape = _lib.make_shape(rows // k, d, F, E, k, _lib.DTYPE_BF16)
@@ -91,9 +96,17 @@ def test_small_m_down_two_per_cu_equals_grouped_gemm(cuda_device, d, counts):
     y_perm = torch.empty(rows, d, dtype=torch.bfloat16, device=cuda_device)
     _lib.call("g5moe_expert_down", ops._ptr(t_off), ops._ptr(wd), ops._ptr(y_perm),
               ops._ptr(ws), ctypes.byref(shape), ops._stream(cuda_device))
-    ref = ops.grouped_gemm(h[:rows + ops.ROW_PAD].contiguous(), rows, t_off, wd)
-    torch.cuda.synchronize()
-    assert torch.equal(y_perm, ref)
+    for e0 in range(0, E, 8):
+        part = list(counts[e0:e0 + 8])
+        o0, o1 = int(off[e0]), int(off[e0 + len(part)])
+        a = torch.randn(o1 - o0 + big + ops.ROW_PAD, F, device=cuda_device,
+                        generator=g).to(torch.bfloat16)
+        a[:o1 - o0] = h[o0:o1]
+        _, t_part = _offsets(part + [big], cuda_device)
+        b = torch.cat([wd[e0:e0 + len(part)], wd[:1]])
+        large = ops.grouped_gemm(a, o1 - o0 + big, t_part, b)
+        torch.cuda.synchronize()
+        assert torch.equal(y_perm[o0:o1], large[:o1 - o0]), e0
     e = int(np.argmax(counts))
     o0, o1 = int(off[e]), int(off[e + 1])
     torch.testing.assert_close(y_perm[o0:o1].float(), h[o0:o1].float() @ wd[e].float().T,

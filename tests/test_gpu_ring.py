@@ -81,7 +81,8 @@ def test_ring_gate_up_equals_persistent_tiles(cuda_device, n, d, F, E, k, p):
     keyed on the token and slot)."""
     print(f"ring gate|up n={n} d={d} F={F} E={E} k={k} p={p}", flush=True)
     g = torch.Generator(device=cuda_device).manual_seed(n + d)
-    big = 24000 if d < 768 else 6000
+    # (past ring_wide's rows: d = 128's two n-tiles stay below half the CUs up to 32,768)
+    big = {128: 40000, 256: 24000, 768: 6000}[d]
     r = lambda *s, std=1.0: (torch.randn(*s, device=cuda_device, generator=g) * std).bfloat16()
     x, wr = r(big, d), r(E, d, std=0.05)
     wgu, wd = r(E, 2 * F, d, std=0.02), r(E, d, F, std=0.02)
