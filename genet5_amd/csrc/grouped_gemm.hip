@@ -31,8 +31,10 @@
 // k-step's first half, the other operand's 8 over the second, one after every
 // fourth MFMA.  The DMA path takes about 45 B per clock and CU; all 16 in the
 // second half asked 64 of it and the in-order waves' MFMA streams stalled behind
-// them (36,400 tokens, outputs the same bit for bit: the layer 957 -> 940 us, the
-// training step 3,329 -> 3,281 us; 4,550 tokens 189 -> 187 us).
+// them (outputs the same bit for bit; the layer at 36,400 tokens 957 -> 940 us; down
+// at 17,000 tokens 166 -> 155, dX 312 -> 294, dh 286 -> 278; the inference gate|up at
+// 13,000 256 -> 249, from 1,000 to 9,000 tokens within 1 % of before).  The training
+// gate|up is the same within 2 % either way, 2,048 to 36,400 tokens.
 //
 // Scheduling: expert row counts live on the device (offsets[]); the grid is
 // one workgroup per CU, and each workgroup walks a list of tiles derived from
@@ -1707,7 +1709,8 @@ void launch_persist(unsigned grid, const GemmArgs& a, hipStream_t st) {
 template <int MAXMB, int OCC, int MODE, bool DROP, bool PADA>
 void launch_ring_tiles(const GemmArgs& a, int64_t rows, hipStream_t st) {
   // tiles: sum_e ceil(ceil(cnt_e / 32) / MAXMB) <= rows / (32 MAXMB) + E per column,
-  // and (MODE 4) at most two zero tiles per expert (383 rows at most)
+  // and (MODE 4) at most two zero tiles per expert (384 rows at most, in
+  // tiles of 256)
   const int64_t mt = (rows + 32 * MAXMB - 1) / (32 * MAXMB) + (MODE == 4 ? 3 : 1) * a.n_experts;
   const unsigned grid = unsigned((mt * (a.Nout / 128) + 7) / 8 * 8);
   hipLaunchKernelGGL((grouped_gemm_ring_kernel<MAXMB, OCC, MODE, DROP, PADA>), dim3(grid),
