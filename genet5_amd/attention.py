@@ -84,7 +84,9 @@ def attn_varlen_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     against the ALiBi distance), and (b) uses a fixed per-query reference maximum
     instead of the online running maximum where the bounds keep every score term
     within 32 of zero (base 2).  The result equals the plain online computation over
-    every block (key_bounds=False) to fp32 rounding of the probabilities."""
+    every block (key_bounds=False) to fp32 rounding of the probabilities.  Calls without
+    alibi_slopes and with max_seqlen <= 2,048 leave the pre-pass out (nothing to skip, and
+    it costs about what the other loop gains)."""
     dev = _check_device(q)
     T, H = q.shape[0], q.shape[1]
     Hkv = k.shape[1] if k.dim() == 3 else -1

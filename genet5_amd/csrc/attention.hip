@@ -18,14 +18,15 @@
 // blocks as runs of one kind (before its queries, across them, after them, the
 // partial last one), so that the block loops carry no branches.
 //
-// What bounds it: with two waves per SIMD the matrix core and the VALU are each
-// busy about half of the cycles and the clock falls to 1.9 GHz under the power
-// limit; per 64-key block and wave 22 MFMAs (704 cycles) against 32 exps (8
-// cycles each), 32 multiplies, 16 conversions and about 30 more.  At 8 x 4,550
-// tokens, 12 heads (captured loops, one GPU, against the register-staged,
-// branching loop with a multiplied-out bias before it): ALiBi 449 -> 377 us, with
-// twice the scores (online loop) 534 -> 453, no ALiBi 745 -> 591 (861 TFLOP/s) and
-// 789 -> 652; 2 x 2,275 without ALiBi 66 -> 49.
+// What bounds it: issue and power.  With two waves per SIMD the matrix core and the
+// VALU are each busy half of the cycles with ALiBi (counters, 8 x 4,550 tokens, 12
+// heads: 50 and 51 %, at 1.98 GHz) and 60 and 57 % without (1.84 GHz under the power
+// limit), no LDS bank conflicts; per 64-key block and wave 22 MFMAs (704 cycles)
+// against 32 exps (8 cycles each), 32 multiplies, 16 conversions and about 30 more.
+// Against the register-staged loop with a branch per block before it (and a
+// multiplied-out bias in its online loop), the same calls on one GPU: 8 x 4,550
+// tokens with ALiBi 402 -> 339 us, with twice the scores (online loop) 522 -> 456, no
+// ALiBi 745 -> 592 (859 TFLOP/s); 2 x 3,000 without ALiBi 115 -> 86, 4 x 2,048 86 -> 74.
 //
 // MFMA layout (v_mfma_f32_32x32x16_bf16): scores are formed transposed,
 // S^T = K . Q^T, with the key block as the A operand and the wave's queries as
@@ -626,10 +627,18 @@ hipError_t launch_attn_fwd(const uint16_t* q, const uint16_t* k, const uint16_t*
                            float* lse, float* kmax_ws, const g5moe_attn_shape& s,
                            hipStream_t st) {
   // Key-norm bounds: block skipping (with ALiBi) and the reference-max loop.  The
-  // pre-pass costs a launch and a pass over k, about 4 us, which short sequences
-  // without ALiBi (nothing to skip) do not earn back: with it against without, 12
-  // heads, 12 sequences up to 1,499 tokens 53.8 against 47.5 us, 2 x 2,275 49.2
-  // against 51.8; with ALiBi 2 x 1,024 20.7 against 19.6, 4,550 60 against 101.
+  // pre-pass is a launch and a read of k, 2-4 us for one sequence.  With the pass
+  // against without, 12 heads, queries and keys N(0, 1), in brackets twice that (the
+  // bounds then leave the online loop in place):
+  //   ALiBi:  1 x 512 12.9, 11.0 (14.7, 11.1); 2 x 1,024 19.8, 19.4 (23.0, 19.6);
+  //           8 x 1,024 43.6, 45.2 (49.2, 47.0); 1 x 4,550 57, 95 (81, 96)
+  //   none:   1 x 512 11.9, 10.0 (13.7, 10.2); 4 x 1,536 52, 55 (58, 53);
+  //           16 x 2,048 264, 286 (299, 288); 2 x 3,000 85, 93 (99, 94);
+  //           8 x 4,550 594, 650 (674, 662)
+  // So without ALiBi the scores, which the host cannot see, decide from about 1,500
+  // tokens on; up to 2,048 the pass is left out.  With ALiBi the length of what is
+  // skipped decides, and short calls keep the pass too: their outputs stay those of
+  // the loop they always took.
   const bool bounds = kmax_ws != nullptr && s.total_tokens > 0 &&
                       (slopes != nullptr || s.max_seqlen > 2048);
   const int n_kblk = int((s.total_tokens + 63) / 64);
