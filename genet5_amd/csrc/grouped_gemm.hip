@@ -1249,9 +1249,13 @@ __global__ __launch_bounds__(256) void grouped_gemm_persist_kernel(GemmArgs args
 // the rows.  One
 // workgroup per tile, one (OCC = 1) or two (OCC = 2) to a CU; all of its LDS is a
 // ring of k-stages (MB = 1: 20 KB each), so up to seven are in flight; fragments
-// are read one 16-k substep ahead.  The weight stream (each weight row read once
-// per m-tile, from beyond the L2) bounds MB = 1, the LDS fragment reads
-// (MB + 1 per MB MFMAs and wave) MB = 4: about 0.25 + 0.1 MB us a k-step.
+// are read one 16-k substep ahead.  MB = 1 is bound by the weight stream, each
+// weight row read once per m-tile from beyond the L2 (down at 300 tokens 85 MB in
+// 24.7 us, 3.4 TB/s); from MB = 2 on by the latency of the stages in flight: the
+// matrix cores are busy 19 % of the cycles and the waves wait 27 % of theirs at MB =
+// 4 with all of the LDS (2,048 tokens), 27 and 52 % with two stages of half of it
+// (4,550), LDS reads under a fifth of the cycles (counters).  The time of a k-step
+// by height and occupancy is in in_place_tile's table.
 // Every accumulator takes its k in the persistent kernel's order, so the outputs
 // are the same bit for bit.
 //
