@@ -1,5 +1,6 @@
 """The grouped GEMM's ring kernel (few rows: tiles of 1 to 4 blocks of 32 rows by 128
-columns) against the persistent 256-row tiles, which serve the launches with many rows.
+columns) and its launches of few persistent tiles against many persistent 256-row tiles,
+which serve the launches with many rows.
 
 Every accumulator takes its k in one order whatever the tile, so the two must agree bit
 for bit; the persistent kernel is checked against float32 products elsewhere
@@ -34,6 +35,11 @@ def _offsets(counts, dev):
     (256, 768, [256, 255, 257, 0, 1, 128, 129, 300, 511, 512, 385, 320, 290, 230, 270]),  # 4, one
     (128, 768, [375, 384, 385, 0, 31, 33, 512, 513, 400, 390, 700, 640, 641, 128, 129]),  # 4, two
     (768, 2304, [2048]),                    # 4, two: one expert
+    # persistent tiles with less than one per CU (whole ones, n-halves), three and two
+    # fragment slots, 256 and 128 columns
+    (192, 768, [800, 769, 0, 1023, 1024, 1025, 700, 1, 900, 850, 760, 513, 640, 1100, 1300]),
+    (448, 256, [9000, 8000, 7000, 9500, 1, 0, 4000, 257]),
+    (384, 640, [9000, 1, 0, 257, 300]),
 ])
 @pytest.mark.parametrize("packed", [False, True])
 def test_ring_equals_persistent_tiles(cuda_device, K, n_out, counts, packed):
